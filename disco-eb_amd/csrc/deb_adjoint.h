@@ -33,31 +33,6 @@ using TD = dn<1 + MAXDIR>;          // (a or tau, theta_1..theta_MAXDIR)
 // device-assembly test of the build checks this for every outlined function.
 #define DEB_OUTLINE __device__ __noinline__
 
-// Rodas5 tableau in flattened form (constant memory, read with wave-uniform
-// indices): stage point u_i = y0 + sum_j kA[i][j] k_j, y1 = y0 + sum_j kA8[j] k_j,
-// stage time t0 + kc[i] h, kd[i] h dT added in stage i, kC[i][j] / h k_j.
-__constant__ double kA[8][8] = {
-    {0, 0, 0, 0, 0, 0, 0, 0},
-    {R5::a21, 0, 0, 0, 0, 0, 0, 0},
-    {R5::a31, R5::a32, 0, 0, 0, 0, 0, 0},
-    {R5::a41, R5::a42, R5::a43, 0, 0, 0, 0, 0},
-    {R5::a51, R5::a52, R5::a53, R5::a54, 0, 0, 0, 0},
-    {R5::a61, R5::a62, R5::a63, R5::a64, R5::a65, 0, 0, 0},
-    {R5::a61, R5::a62, R5::a63, R5::a64, R5::a65, 1.0, 0, 0},
-    {R5::a61, R5::a62, R5::a63, R5::a64, R5::a65, 1.0, 1.0, 0}};
-__constant__ double kA8[8] = {R5::a61, R5::a62, R5::a63, R5::a64, R5::a65, 1.0, 1.0, 1.0};
-__constant__ double kC[8][8] = {
-    {0, 0, 0, 0, 0, 0, 0, 0},
-    {R5::C21, 0, 0, 0, 0, 0, 0, 0},
-    {R5::C31, R5::C32, 0, 0, 0, 0, 0, 0},
-    {R5::C41, R5::C42, R5::C43, 0, 0, 0, 0, 0},
-    {R5::C51, R5::C52, R5::C53, R5::C54, 0, 0, 0, 0},
-    {R5::C61, R5::C62, R5::C63, R5::C64, R5::C65, 0, 0, 0},
-    {R5::C71, R5::C72, R5::C73, R5::C74, R5::C75, R5::C76, 0, 0},
-    {R5::C81, R5::C82, R5::C83, R5::C84, R5::C85, R5::C86, R5::C87, 0}};
-__constant__ double kc[8] = {0.0, R5::c2, R5::c3, R5::c4, R5::c5, 1.0, 1.0, 1.0};
-__constant__ double kd[8] = {R5::d1, R5::d2, R5::d3, R5::d4, R5::d5, 0.0, 0.0, 0.0};
-
 // ---------------------------------------------------------------------------
 // cross-lane moves and reductions of composite scalars, component by
 // component (member access only)
@@ -897,9 +872,7 @@ __device__ __forceinline__ TD seed_td(double v, double d0) {
 }
 
 // one forward step from (t0, y0) to y1, its eight stage vectors stored in
-// K[8][NS][64] (inlined, with its factorisation, right-hand sides and solves
-// as calls: the whole step as one call is large enough to need long branches,
-// which must stay out of non-kernel functions)
+// K[8][NS][64]
 template <int NS>
 __device__ __forceinline__ void step_store(Mode<NS> &m, Ctx &cx, double t0, double h, const double (&y0)[NS],
                                            double (&y1)[NS], double *K, lds_double *kl) {
@@ -909,7 +882,7 @@ __device__ __forceinline__ void step_store(Mode<NS> &m, Ctx &cx, double t0, doub
 #pragma unroll
     for (int s = 0; s < NS; ++s) K[(i * NS + s) * WAVE + lane] = k[s];
   };
-  rodas5_step_s<NS, decltype(store), true>(m, cx, t0, h, y0, y1, err, store, kl);
+  rodas5_step_s<NS>(m, cx, t0, h, y0, y1, err, store, kl);
 }
 
 // ---------------------------------------------------------------------------
@@ -1352,6 +1325,7 @@ __device__ __forceinline__ void adjoint_mode(const Params<NS> &P, const AdjArgs 
   m.u = (lds_mode_u *)&mu;
 #pragma unroll
   for (int s = 0; s < NS; ++s) m.rd[s] = P.rowdesc[s][lane];
+  row_consts<NS>(m.rd, cx, m.rk);
   m.nlev = mode_levels(P.cfg, P.nq);
   const double *tout = P.tau_out + (long long)ci * P.nout;
   const double *dtout = A.dtau + (long long)ci * A.ndir * P.nout;
@@ -1399,6 +1373,13 @@ __device__ __forceinline__ void adjoint_mode(const Params<NS> &P, const AdjArgs 
     // forward again over the segment from its checkpoint: states and stage
     // vectors into the ring
     {
+      // the step factors of the recompute are its own: they stay in registers,
+      // where those of the reversal live in memory across its calls
+      Mode<NS> mr;
+      mr.pcr = pcr;
+      mr.u = (lds_mode_u *)&mu;
+      mr.rk = m.rk;
+      mr.nlev = m.nlev;
       double y[NS], y1[NS];
       const double *yc = chunk_y(chunk);
 #pragma unroll
@@ -1407,7 +1388,7 @@ __device__ __forceinline__ void adjoint_mode(const Params<NS> &P, const AdjArgs 
         double *ry = ring_y(j);
 #pragma unroll
         for (int s = 0; s < NS; ++s) ry[s * WAVE + lane] = y[s];
-        step_store<NS>(m, cx, tt[j], tt[j + 1] - tt[j], y, y1, ring_k(j), (lds_double *)KBl);
+        step_store<NS>(mr, cx, tt[j], tt[j + 1] - tt[j], y, y1, ring_k(j), (lds_double *)KBl);
 #pragma unroll
         for (int s = 0; s < NS; ++s) y[s] = y1[s];
       }

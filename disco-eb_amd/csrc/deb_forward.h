@@ -301,6 +301,7 @@ __device__ __forceinline__ void integrate_mode(const Params<NS> &P, int ci, int 
   m.u = (lds_mode_u *)&mu;
 #pragma unroll
   for (int s = 0; s < NS; ++s) m.rd[s] = P.rowdesc[s][lane];
+  row_consts<NS>(m.rd, cx, m.rk);
   m.nlev = mode_levels(P.cfg, P.nq);
   // stage vectors in the kernel's LDS (lds holds fwd_lds_doubles<NS>())
   lds_double *const kl = stage_in_lds<NS>() ? (lds_double *)lds : nullptr;
@@ -419,6 +420,7 @@ __device__ __forceinline__ void integrate_batch(const Params<NS> &P, int ci, int
   m.u = (lds_mode_u *)&mu;
 #pragma unroll
   for (int s = 0; s < NS; ++s) m.rd[s] = P.rowdesc[s][lane];
+  row_consts<NS>(m.rd, cx, m.rk);
   m.nlev = mode_levels(P.cfg, P.nq);
   // stage vectors in the kernel's LDS (lds holds fwd_lds_doubles<NS>())
   lds_double *const kl = stage_in_lds<NS>() ? (lds_double *)lds : nullptr;
@@ -470,6 +472,7 @@ __device__ __forceinline__ void integrate_batch(const Params<NS> &P, int ci, int
       const double *src = state(b, 0);
 #pragma unroll
       for (int s = 0; s < NS; ++s) y[s] = src[s * WAVE];
+      row_consts<NS>(m.rd, cx, m.rk);
       rodas5_step<NS>(m, cx, tprev, dt, y, y1, err, kl);
       // error-norm weights: indices (a, eta, delta_c, delta_b, theta_b, delta_gamma) of slot 0
       double ew = 0.0;

@@ -113,7 +113,9 @@ __global__ void __launch_bounds__(WAVE) deb_rhs_kernel(const Params<NS> P, const
     rd[s] = P.rowdesc[s][lane];
     y[s] = rd_type(rd[s]) != R_NONE ? src[rd_idx(rd[s])] : 0.0;
   }
-  eval_rhs<NS, double>(cx, rd, H.t0[item], y, f);
+  RowK<NS> K;
+  row_consts<NS>(rd, cx, K);
+  eval_rhs<NS, double>(cx, K, H.t0[item], y, f);
   double *dst = H.y1 + (int64_t)item * P.n;
 #pragma unroll
   for (int s = 0; s < NS; ++s)
@@ -122,6 +124,7 @@ __global__ void __launch_bounds__(WAVE) deb_rhs_kernel(const Params<NS> P, const
 
 template <int NS>
 __global__ void __launch_bounds__(WAVE) deb_step_kernel(const Params<NS> P, const HookArgs<NS> H) {
+  __shared__ double lds[fwd_lds_doubles<NS>()];
   __shared__ double pcr[pcr_lds_doubles<NS>()];
   const int item = blockIdx.x;
   if (item >= H.m) return;
@@ -148,8 +151,9 @@ __global__ void __launch_bounds__(WAVE) deb_step_kernel(const Params<NS> P, cons
     m.rd[s] = P.rowdesc[s][lane];
     y[s] = rd_type(m.rd[s]) != R_NONE ? src[rd_idx(m.rd[s])] : 0.0;
   }
+  row_consts<NS>(m.rd, cx, m.rk);
   const double t0 = H.t0[item];
-  rodas5_step<NS>(m, cx, t0, H.t1[item] - t0, y, y1, err);
+  rodas5_step<NS>(m, cx, t0, H.t1[item] - t0, y, y1, err, stage_in_lds<NS>() ? (lds_double *)lds : nullptr);
   double *d1 = H.y1 + (int64_t)item * P.n;
   double *de = H.err + (int64_t)item * P.n;
 #pragma unroll

@@ -554,4 +554,159 @@ __device__ __forceinline__ Coef<T> row_coef_slot(uint32_t d, const Bg<T> &b, con
   else return row_coef<T>(d, b, cx, invtau);
 }
 
+// ---------------------------------------------------------------------------
+// The rows as constants times background features.  Along one mode every
+// coefficient of a row is a number that depends on the row, k and the
+// cosmology only, times one of a few wave-uniform functions of a (the opacity,
+// aH, 1/a, ...) and, on massive-nu rows, the bin velocity: the numbers are
+// formed once per mode (row_consts) and a right-hand side costs about a dozen
+// multiplications per slot, where the selects of row_coef_wave took about two
+// hundred instructions.  The same products as row_visit up to the order of the
+// factors.
+template <int NS>
+struct RowK {
+  double sub[NS], sup[NS];             // neighbours (times v_q on massive-nu rows)
+  double ph[NS];                       // 1 on photon rows (-opac on the diagonal)
+  double tr[NS];                       // l + 1 on truncation rows, else 0
+  double uh[NS], ueta[NS], upi[NS];    // where h', eta', Pi enter (upi times opac)
+  double ch[NS], ceta[NS], cpi[NS];    // contributions to h', eta', Pi
+  double aq[NS];                       // m_nu / q on massive-nu rows, else 0
+  double leaf, dah;                    // slot 0: leaf coupling, -aH on the diagonal
+  uint32_t qmask;                      // slots that hold massive-nu rows (wave-uniform)
+};
+
+template <int NS>
+__device__ __forceinline__ void row_consts(const uint32_t (&rd)[NS], const Ctx &cx, RowK<NS> &K) {
+  const int lane = lane_id();
+  const deb_cosmo_t &c = *cx.c;
+  const double k = cx.k, k2 = k * k, hk2 = 0.5 / k2;
+  K.qmask = 0;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const uint32_t t = rd_type(rd[s]);
+    const double l = (double)rd_l(rd[s]);
+    const bool F2 = t == R_F2, FL = t == R_FL, FLM = t == R_FLMAX, G0 = t == R_G0, GL = t == R_GL, G2 = t == R_G2,
+               GLM = t == R_GLMAX, DR = t == R_DR, TR = t == R_TR, FR2 = t == R_FR2, FRL = t == R_FRL,
+               FRLM = t == R_FRLMAX, Q0 = t == R_Q0, Q1 = t == R_Q1, Q2 = t == R_Q2, QL = t == R_QL,
+               QLM = t == R_QLMAX;
+    const bool qrow = t >= R_Q0 && t <= R_QLMAX;
+    const int qi = qrow ? (int)rd_q(rd[s]) : 0;
+    const double wq = cx.w[qi], dl = cx.dlnf[qi];
+    const double il = rcp_nr(2.0 * l + 1.0);
+    const bool mid = FL || GL || FRL || QL, last = FLM || GLM || FRLM || QLM;
+    double v = 0.0;
+    v = mid ? k * (l * il) : v;
+    v = last ? k : v;
+    v = (G2 || Q2) ? 0.4 * k : v;
+    v = Q1 ? k * (1.0 / 3.0) : v;
+    v = (F2 || FR2) ? 8.0 / 15.0 : v;
+    K.sub[s] = TR ? 0.25 * k2 : v;
+    v = 0.0;
+    v = (F2 || G2 || FR2 || Q2) ? -(0.6 * k) : v;
+    v = mid ? -(k * ((l + 1.0) * il)) : v;
+    v = (G0 || Q0) ? -k : v;
+    v = Q1 ? -(k * (2.0 / 3.0)) : v;
+    v = DR ? -4.0 / 3.0 : v;
+    K.sup[s] = TR ? -0.5 * k2 : v;
+    K.ph[s] = (F2 || FL || FLM || G0 || GL || G2 || GLM) ? 1.0 : 0.0;
+    K.tr[s] = last ? l + 1.0 : 0.0;
+    v = (F2 || FR2) ? 4.0 / 15.0 : 0.0;
+    v = DR ? -2.0 / 3.0 : v;
+    v = Q0 ? dl * (1.0 / 6.0) : v;
+    K.uh[s] = Q2 ? dl * (-1.0 / 15.0) : v;
+    K.ueta[s] = (F2 || FR2) ? 8.0 / 5.0 : (Q2 ? -0.4 * dl : 0.0);
+    K.upi[s] = (F2 || G2) ? 0.1 : (G0 ? 0.5 : 0.0);
+    K.ch[s] = DR ? c.grhor * c.Neff : (Q0 ? c.grhor * c.Nmnu * wq : 0.0);
+    K.ceta[s] = TR ? (4.0 / 3.0) * c.Neff * c.grhor * hk2 : (Q1 ? c.Nmnu * c.grhor * k * wq * hk2 : 0.0);
+    K.cpi[s] = (F2 || G0 || G2) ? 1.0 : 0.0;
+    K.aq[s] = qrow ? c.amnu * rcp_nr(cx.q[qi]) : 0.0;
+    if (__ballot(qrow) != 0) K.qmask |= 1u << s;
+    if (s == 0) {
+      const double rc = c.grhom * (c.Omegam - c.Omegab), rb = c.grhom * c.Omegab;
+      const bool DC = lane == L_DC, DB = lane == L_DB, TC = lane == L_TC, TB = lane == L_TB, DG = lane == L_DG,
+                 TG = lane == L_TG, ETA = lane == L_ETA;
+      K.sup[0] = (DC || DB) ? -1.0 : (TG ? -0.5 * k2 : K.sup[0]);
+      K.ph[0] = TG ? 1.0 : K.ph[0];
+      K.uh[0] = (DC || DB) ? -0.5 : (DG ? -2.0 / 3.0 : K.uh[0]);
+      K.ueta[0] = ETA ? 1.0 : K.ueta[0];
+      v = ETA ? 2.0 * k2 : K.ch[0];
+      v = DC ? rc : v;
+      v = DB ? rb : v;
+      K.ch[0] = DG ? c.grhog : v;
+      v = TC ? rc * hk2 : K.ceta[0];
+      v = TB ? rb * hk2 : v;
+      K.ceta[0] = TG ? (4.0 / 3.0) * c.grhog * hk2 : v;
+      K.leaf = DG ? -4.0 / 3.0 : (TG ? 0.25 * k2 : 0.0);
+      v = (TC || TB) ? 1.0 : 0.0;
+      K.dah = (lane == L_TQ && !cx.lambda) ? 1.0 - 3.0 * c.cs2_DE : v;
+    }
+  }
+}
+
+// v_q = (1 + x^2)^(-1/2) and 1/v_q of x = a m_nu / q
+__device__ __forceinline__ void bin_velocity(double a, double aq, double &vq, double &ivq) {
+  const double x = a * aq, s2 = 1.0 + x * x;
+  vq = rsq_nr(s2);
+  ivq = s2 * vq;
+}
+__device__ __forceinline__ void bin_velocity(dual a, double aq, dual &vq, dual &ivq) {
+  const double x = a.v * aq, s2 = 1.0 + x * x, hd = x * (aq * a.d);
+  vq.v = rsq_nr(s2);
+  ivq.v = s2 * vq.v;
+  ivq.d = hd * vq.v;
+  vq.d = -hd * (vq.v * vq.v * vq.v);
+}
+
+// the coefficients of slot s's rows at background b, from their constants
+template <int NS, typename T>
+__device__ __forceinline__ Coef<T> row_lin(const RowK<NS> &K, int s, const Bg<T> &b, const Ctx &cx, double invtau) {
+  Coef<T> r;
+  T vq = tconst<T>(1.0), ivq = tconst<T>(1.0);
+  if ((K.qmask >> s) & 1u) bin_velocity(b.a, K.aq[s], vq, ivq);
+  r.sub = K.sub[s] * vq;
+  r.sup = K.sup[s] * vq;
+  r.diag = -(K.ph[s] * b.opac) - K.tr[s] * invtau;
+  r.uh = tconst<T>(K.uh[s]);
+  r.ueta = tconst<T>(K.ueta[s]);
+  r.upi = K.upi[s] * b.opac;
+  r.cpi = tconst<T>(K.cpi[s]);
+  r.leaf = tconst<T>(0.0);
+  const T gh = b.ia2 * b.iaH;
+  r.ch = K.ch[s] * (ivq * gh);
+  r.ceta = K.ceta[s] * b.ia2;
+  r.c1 = (-K.ch[s]) * ((ivq + vq) * b.ia);
+  if (s == 0) {
+    const int lane = lane_id();
+    const double k2 = cx.k * cx.k;
+    const bool dcb = lane == L_DC || lane == L_DB, eta = lane == L_ETA, tb = lane == L_TB, tg = lane == L_TG;
+    const T po = b.pb43 * b.opac;
+    r.leaf = tconst<T>(K.leaf);
+    r.diag = r.diag - K.dah * b.aH;
+    r.diag = tb ? r.diag - po : r.diag;
+    r.sub = tb ? k2 * b.cs2 : (tg ? b.opac : r.sub);
+    r.sup = tb ? po : r.sup;
+    r.ch = (dcb || eta) ? K.ch[0] * (eta ? b.iaH : b.ia * b.iaH) : r.ch;
+    r.c1 = (dcb || eta) ? tconst<T>(eta ? 0.0 : -K.ch[0]) : r.c1;
+    r.ceta = (tb || lane == L_TC) ? K.ceta[0] * b.ia : r.ceta;
+    // dark-energy fluid (frozen for a cosmological constant)
+    if (!cx.lambda) {
+      const double cs2Q = cx.c->cs2_DE, gde = cx.c->grhom * cx.c->OmegaDE;
+      const double ik2 = 1.0 / k2;
+      const T opw = 1.0 + b.w;
+      const T rq = gde * b.rhoQ * (b.a * b.a);
+      const bool dq = lane == L_DQ, tq = lane == L_TQ;
+      const T dc = cs2Q - b.ca2;
+      r.diag = dq ? -3.0 * (cs2Q - b.w) * b.aH : r.diag;
+      r.sup = dq ? -opw - 9.0 * opw * dc * b.aH * b.aH * ik2 : r.sup;
+      r.uh = dq ? -0.5 * opw : r.uh;
+      r.ch = dq ? rq * b.iaH : r.ch;
+      r.sub = tq ? cs2Q / opw * k2 : r.sub;
+      r.ceta = tq ? opw * rq * (0.5 * ik2) : r.ceta;
+      const T q1 = rq + 3.0 * cs2Q * rq, q2 = 3.0 * dc * (3.0 * b.aH * ik2) * opw * rq;
+      r.c1 = (dq || tq) ? -b.a * (dq ? q1 : q2) : r.c1;
+    }
+  }
+  return r;
+}
+
 }  // namespace deb

@@ -28,6 +28,7 @@ typedef DEB_LDS ModeU lds_mode_u;
 template <int NS>
 struct Mode {
   uint32_t rd[NS];
+  RowK<NS> rk;       // the rows' constants (row_consts)
   // PCR factors of W_B: d' = sig*d + al*d[i-s] + be*d[i+s] at level s = 2^L;
   // al and be live in the wave's LDS ([PCR_LEVELS][2][NS][64], pcr_lds_doubles)
   lds_double *pcr;
@@ -50,7 +51,7 @@ struct Mode {
 
 // evaluate f (T-valued) at (tau, y); optionally return the coefficient rows
 template <int NS, typename T>
-__device__ __forceinline__ void eval_rhs(Ctx &cx, const uint32_t (&rd)[NS], double tau, const double (&y)[NS],
+__device__ __forceinline__ void eval_rhs(Ctx &cx, const RowK<NS> &K, double tau, const double (&y)[NS],
                                          T (&f)[NS], Coef<T> (*co)[NS] = nullptr, T *aH_out = nullptr) {
   const int lane = lane_id();
   double a0 = readlane(y[0], L_A);
@@ -60,13 +61,7 @@ __device__ __forceinline__ void eval_rhs(Ctx &cx, const uint32_t (&rd)[NS], doub
   const double invtau = 1.0 / tau;
   Coef<T> cf[NS];
 #pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    // five slots (lmax 50) keep the switch: there the stage vectors stay in
-    // registers, and the selects' extra live values cost more than the
-    // branches they save
-    if constexpr (NS <= 4) cf[s] = row_coef_slot<T>(rd[s], b, cx, invtau, s == 0);
-    else cf[s] = row_coef<T>(rd[s], b, cx, invtau);
-  }
+  for (int s = 0; s < NS; ++s) cf[s] = row_lin<NS, T>(K, s, b, cx, invtau);
   // functionals h', eta', Pi, f_1
   constexpr int NV = (sizeof(T) == sizeof(double)) ? 4 : 8;
   double part[NV];
@@ -122,14 +117,10 @@ __device__ __forceinline__ void eval_rhs(Ctx &cx, const uint32_t (&rd)[NS], doub
 
 // df/dtau: only the hierarchy truncation rows depend on tau explicitly
 template <int NS>
-__device__ __forceinline__ void dfdtau(const uint32_t (&rd)[NS], double tau, const double (&y)[NS], double (&dT)[NS]) {
+__device__ __forceinline__ void dfdtau(const RowK<NS> &K, double tau, const double (&y)[NS], double (&dT)[NS]) {
   const double it = 1.0 / tau, it2 = it * it;
 #pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    uint32_t t = rd_type(rd[s]);
-    bool trunc = (t == R_FLMAX) | (t == R_GLMAX) | (t == R_FRLMAX) | (t == R_QLMAX);
-    dT[s] = trunc ? (rd_l(rd[s]) + 1.0) * it2 * y[s] : 0.0;
-  }
+  for (int s = 0; s < NS; ++s) dT[s] = K.tr[s] != 0.0 ? K.tr[s] * it2 * y[s] : 0.0;
 }
 
 // W_B^{-1} r (leaf elimination + PCR)
@@ -164,14 +155,17 @@ __device__ __forceinline__ void bsolve(const Mode<NS> &m, double (&x)[NS]) {
   if (lane == L_DG) x[0] = (rdg - m.u->wdg * xtg) * m.u->ddg;
 }
 
-// factorisation of W at (tau0, y0) for step size h
+// factorisation of W at (tau0, y0) for step size h; f0 = f(tau0, y0)
 template <int NS>
-__device__ __forceinline__ void factor(Mode<NS> &m, Ctx &cx, double tau0, const double (&y0)[NS], double h) {
+__device__ __forceinline__ void factor(Mode<NS> &m, Ctx &cx, double tau0, const double (&y0)[NS], double h,
+                                       double (&f0)[NS]) {
   const int lane = lane_id();
   constexpr double gamma = 0.19;
   dual fd[NS];
   Coef<dual> co[NS];
-  eval_rhs<NS, dual>(cx, m.rd, tau0, y0, fd, &co);
+  eval_rhs<NS, dual>(cx, m.rk, tau0, y0, fd, &co);
+#pragma unroll
+  for (int s = 0; s < NS; ++s) f0[s] = fd[s].v;
   m.u->gh = gamma * h;
   const double igh = 1.0 / m.u->gh;
   double gprime = readlane(fd[0].d, L_A);
@@ -180,8 +174,8 @@ __device__ __forceinline__ void factor(Mode<NS> &m, Ctx &cx, double tau0, const 
   double A[NS], Bd[NS], Cc[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    uint32_t t = rd_type(m.rd[s]);
-    bool special = (t == R_NONE) | (t == R_A) | (t == R_AHP);
+    // the a-row and the a*h' row are solved apart (unused lanes hold zero rows)
+    const bool special = s == 0 && lane <= L_AHP;
     m.jcol[s] = special ? 0.0 : fd[s].d;
     A[s] = special ? 0.0 : -co[s].sub.v;
     Cc[s] = special ? 0.0 : -co[s].sup.v;
@@ -251,8 +245,7 @@ __device__ __forceinline__ void factor(Mode<NS> &m, Ctx &cx, double tau0, const 
     double x[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      uint32_t t = rd_type(m.rd[s]);
-      bool special = (t == R_NONE) | (t == R_A) | (t == R_AHP);
+      const bool special = s == 0 && lane <= L_AHP;
       double u = r == 0 ? co[s].uh.v : (r == 1 ? co[s].ueta.v : co[s].upi.v);
       x[s] = special ? 0.0 : u;
     }
@@ -350,152 +343,133 @@ struct R5 {
                           d4 = 0.3449828624725343, d5 = -0.377417564392089818;
 };
 
-// Out-of-line versions of the factorisation and the right-hand side, for
-// kernels that run the step next to much other live state (the reverse
-// kernel): as calls, the step factors stay in memory instead of registers.
+// Out-of-line factorisation, for the reverse of a step (next to much other
+// live state): as a call, the step factors stay in memory instead of registers.
 template <int NS>
 __device__ __noinline__ void factor_call(Mode<NS> &m, Ctx &cx, double tau0, const double (&y0)[NS], double h) {
-  factor<NS>(m, cx, tau0, y0, h);
-}
-// (the calls work on private copies of their array arguments: stores through
-// the references could alias the inputs as far as the compiler knows, which
-// would reload them from the caller's frame after every store)
-template <int NS>
-__device__ __noinline__ void rhs_call(Ctx &cx, const uint32_t (&rd)[NS], double tau, const double (&y_in)[NS],
-                                      double (&f_out)[NS]) {
-  double y[NS], f[NS];
-  uint32_t d[NS];
-#pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    y[s] = y_in[s];
-    d[s] = rd[s];
-  }
-  eval_rhs<NS, double>(cx, d, tau, y, f);
-#pragma unroll
-  for (int s = 0; s < NS; ++s) f_out[s] = f[s];
+  double f0[NS];
+  factor<NS>(m, cx, tau0, y0, h, f0);
 }
 
+// Rodas5 tableau in flattened form (constant memory, read with wave-uniform
+// indices): stage point u_i = y0 + sum_j kA[i][j] k_j, y1 = y0 + sum_j kA8[j] k_j,
+// stage time t0 + kc[i] h, kd[i] h dT added in stage i, kC[i][j] / h k_j.
+__constant__ double kA[8][8] = {
+    {0, 0, 0, 0, 0, 0, 0, 0},
+    {R5::a21, 0, 0, 0, 0, 0, 0, 0},
+    {R5::a31, R5::a32, 0, 0, 0, 0, 0, 0},
+    {R5::a41, R5::a42, R5::a43, 0, 0, 0, 0, 0},
+    {R5::a51, R5::a52, R5::a53, R5::a54, 0, 0, 0, 0},
+    {R5::a61, R5::a62, R5::a63, R5::a64, R5::a65, 0, 0, 0},
+    {R5::a61, R5::a62, R5::a63, R5::a64, R5::a65, 1.0, 0, 0},
+    {R5::a61, R5::a62, R5::a63, R5::a64, R5::a65, 1.0, 1.0, 0}};
+__constant__ double kA8[8] = {R5::a61, R5::a62, R5::a63, R5::a64, R5::a65, 1.0, 1.0, 1.0};
+__constant__ double kC[8][8] = {
+    {0, 0, 0, 0, 0, 0, 0, 0},
+    {R5::C21, 0, 0, 0, 0, 0, 0, 0},
+    {R5::C31, R5::C32, 0, 0, 0, 0, 0, 0},
+    {R5::C41, R5::C42, R5::C43, 0, 0, 0, 0, 0},
+    {R5::C51, R5::C52, R5::C53, R5::C54, 0, 0, 0, 0},
+    {R5::C61, R5::C62, R5::C63, R5::C64, R5::C65, 0, 0, 0},
+    {R5::C71, R5::C72, R5::C73, R5::C74, R5::C75, R5::C76, 0, 0},
+    {R5::C81, R5::C82, R5::C83, R5::C84, R5::C85, R5::C86, R5::C87, 0}};
+__constant__ double kc[8] = {0.0, R5::c2, R5::c3, R5::c4, R5::c5, 1.0, 1.0, 1.0};
+__constant__ double kd[8] = {R5::d1, R5::d2, R5::d3, R5::d4, R5::d5, 0.0, 0.0, 0.0};
+
 // one Rodas5Transformed step (ode_integrators_stiff.py:718-834): y1 and err = k8;
-// st(i, k) sees every stage vector k_{i+1} once it is solved.  CALLS selects
-// the out-of-line factorisation and right-hand side.  With kl (the
-// wave's LDS, 7 x NS x 64 doubles) the stage vectors k1..k7 are kept there
-// instead of in registers, which relieves the register file of the kernels
-// that run the step fully inlined.
-template <int NS, class Store, bool CALLS = false>
+// st(i, k) sees every stage vector k_{i+1} once it is solved.  The stages run
+// as a loop over the tableau: unrolled, the step is about 240 KB of code, four
+// times the instruction cache, and every wave fetched it again each step.
+// Stage 1's right-hand side is the factorisation's.  With kl (the wave's LDS,
+// 7 x NS x 64 doubles) the stage vectors k1..k7 are kept there, else in
+// registers.
+template <int NS, class Store>
 __device__ __forceinline__ void rodas5_step_s(Mode<NS> &m, Ctx &cx, double t0, double dt, const double (&y0)[NS],
                                               double (&y1)[NS], double (&err)[NS], Store st,
                                               lds_double *kl = nullptr) {
-  using R = R5;
   const int lane = lane_id();
-  auto eval_rhs_ = [&](double tau, const double (&y)[NS], double (&f)[NS]) {
-    if constexpr (CALLS) rhs_call<NS>(cx, m.rd, tau, y, f);
-    else eval_rhs<NS, double>(cx, m.rd, tau, y, f);
-  };
-  // the solves stay inline in both forms (as a call each, the recompute of the
-  // reverse kernel measured 2 % slower)
-  auto wsolve_ = [&](double (&r)[NS]) { wsolve<NS>(m, r); };
-  if constexpr (CALLS) factor_call<NS>(m, cx, t0, y0, dt);
-  else factor<NS>(m, cx, t0, y0, dt);
-  double dT[NS];
-  dfdtau<NS>(m.rd, t0, y0, dT);
+  double k[NS], u[NS], f[NS], dT[NS];
+  factor<NS>(m, cx, t0, y0, dt, f);
+  dfdtau<NS>(m.rk, t0, y0, dT);
+  // the stage vectors start from zero: a stage then sums over fixed columns of
+  // the tableau (zero from column i on) without meeting what an earlier step,
+  // possibly one that was rejected for a non-finite error, left behind
   double kr[7][NS];
-  // stage vector i (0-based) of slot s: registers, or LDS when kl is given
-  auto K = [&](int i, int s) -> double { return kl ? (double)kl[(i * NS + s) * WAVE + lane] : kr[i][s]; };
-  auto keep = [&](int i, const double (&k)[NS]) {
+#pragma unroll
+  for (int j = 0; j < 7; ++j)
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      if (kl) kl[(i * NS + s) * WAVE + lane] = k[s];
-      else kr[i][s] = k[s];
+      if (kl) kl[(j * NS + s) * WAVE + lane] = 0.0;
+      else kr[j][s] = 0.0;
     }
-  };
-  double k[NS], u[NS], f[NS];
+  auto K = [&](int j, int s) -> double { return kl ? (double)kl[(j * NS + s) * WAVE + lane] : kr[j][s]; };
   const double idt = 1.0 / dt;
-  // stage 1
-  eval_rhs_(t0, y0, f);
 #pragma unroll
-  for (int s = 0; s < NS; ++s) k[s] = f[s] + dt * R::d1 * dT[s];
-  wsolve_(k);
-  st(0, k);
-  keep(0, k);
-  // stage 2
+  for (int s = 0; s < NS; ++s) {
+    u[s] = y0[s];
+    k[s] = 0.0;
+  }
+#pragma nounroll
+  for (int i = 0; i < 8; ++i) {
+    double ck[NS];
 #pragma unroll
-  for (int s = 0; s < NS; ++s) u[s] = y0[s] + R::a21 * K(0, s);
-  eval_rhs_(t0 + R::c2 * dt, u, f);
+    for (int s = 0; s < NS; ++s) ck[s] = 0.0;
+    if (i > 0) {
+      // u_i, and the sum of the C_ij k_j; from the seventh stage on u_i = u_{i-1} + k_{i-1}
+      double du[NS];
 #pragma unroll
-  for (int s = 0; s < NS; ++s) k[s] = f[s] + dt * R::d2 * dT[s] + (R::C21 * idt) * K(0, s);
-  wsolve_(k);
-  st(1, k);
-  keep(1, k);
-  // stage 3
+      for (int s = 0; s < NS; ++s) du[s] = i >= 6 ? u[s] + k[s] : y0[s];
+      const double la = i >= 6 ? 0.0 : 1.0;
 #pragma unroll
-  for (int s = 0; s < NS; ++s) u[s] = y0[s] + R::a31 * K(0, s) + R::a32 * K(1, s);
-  eval_rhs_(t0 + R::c3 * dt, u, f);
+      for (int j = 0; j < 3; ++j) {
+        const double aij = la * kA[i][j], cij = kC[i][j];
 #pragma unroll
-  for (int s = 0; s < NS; ++s)
-    k[s] = f[s] + dt * R::d3 * dT[s] + ((R::C31 * idt) * K(0, s) + (R::C32 * idt) * K(1, s));
-  wsolve_(k);
-  st(2, k);
-  keep(2, k);
-  // stage 4
+        for (int s = 0; s < NS; ++s) {
+          const double kj = K(j, s);
+          du[s] += aij * kj;
+          ck[s] += cij * kj;
+        }
+      }
+      if (i > 3) {
 #pragma unroll
-  for (int s = 0; s < NS; ++s) u[s] = y0[s] + R::a41 * K(0, s) + R::a42 * K(1, s) + R::a43 * K(2, s);
-  eval_rhs_(t0 + R::c4 * dt, u, f);
+        for (int j = 3; j < 7; ++j) {
+          const double aij = la * kA[i][j], cij = kC[i][j];
 #pragma unroll
-  for (int s = 0; s < NS; ++s)
-    k[s] = f[s] + dt * R::d4 * dT[s] +
-           ((R::C41 * idt) * K(0, s) + (R::C42 * idt) * K(1, s) + (R::C43 * idt) * K(2, s));
-  wsolve_(k);
-  st(3, k);
-  keep(3, k);
-  // stage 5
+          for (int s = 0; s < NS; ++s) {
+            const double kj = K(j, s);
+            if (j < 5) du[s] += aij * kj;
+            ck[s] += cij * kj;
+          }
+        }
+      }
 #pragma unroll
-  for (int s = 0; s < NS; ++s)
-    u[s] = y0[s] + R::a51 * K(0, s) + R::a52 * K(1, s) + R::a53 * K(2, s) + R::a54 * K(3, s);
-  eval_rhs_(t0 + R::c5 * dt, u, f);
+      for (int s = 0; s < NS; ++s) u[s] = du[s];
+      eval_rhs<NS, double>(cx, m.rk, t0 + kc[i] * dt, u, f);
+    }
+    const double hd = dt * kd[i];
 #pragma unroll
-  for (int s = 0; s < NS; ++s)
-    k[s] = f[s] + dt * R::d5 * dT[s] +
-           ((R::C51 * idt) * K(0, s) + (R::C52 * idt) * K(1, s) + (R::C53 * idt) * K(2, s) +
-            (R::C54 * idt) * K(3, s));
-  wsolve_(k);
-  st(4, k);
-  keep(4, k);
-  // stage 6
+    for (int s = 0; s < NS; ++s) k[s] = f[s] + hd * dT[s] + idt * ck[s];
+    wsolve<NS>(m, k);
+    st(i, k);
+    if (kl) {
+      if (i < 7) {
 #pragma unroll
-  for (int s = 0; s < NS; ++s)
-    u[s] = y0[s] + R::a61 * K(0, s) + R::a62 * K(1, s) + R::a63 * K(2, s) + R::a64 * K(3, s) + R::a65 * K(4, s);
-  eval_rhs_(t0 + dt, u, f);
+        for (int s = 0; s < NS; ++s) kl[(i * NS + s) * WAVE + lane] = k[s];
+      }
+    } else {
 #pragma unroll
-  for (int s = 0; s < NS; ++s)
-    k[s] = f[s] + ((R::C61 * idt) * K(0, s) + (R::C62 * idt) * K(1, s) + (R::C63 * idt) * K(2, s) +
-                   (R::C64 * idt) * K(3, s) + (R::C65 * idt) * K(4, s));
-  wsolve_(k);
-  st(5, k);
-  keep(5, k);
-  // stage 7
+      for (int j = 0; j < 7; ++j)
+        if (i == j) {
 #pragma unroll
-  for (int s = 0; s < NS; ++s) u[s] = u[s] + k[s];
-  eval_rhs_(t0 + dt, u, f);
+          for (int s = 0; s < NS; ++s) kr[j][s] = k[s];
+        }
+    }
+  }
 #pragma unroll
-  for (int s = 0; s < NS; ++s)
-    k[s] = f[s] + ((R::C71 * idt) * K(0, s) + (R::C72 * idt) * K(1, s) + (R::C73 * idt) * K(2, s) +
-                   (R::C74 * idt) * K(3, s) + (R::C75 * idt) * K(4, s) + (R::C76 * idt) * K(5, s));
-  wsolve_(k);
-  st(6, k);
-  keep(6, k);
-  // stage 8
-#pragma unroll
-  for (int s = 0; s < NS; ++s) u[s] = u[s] + k[s];
-  eval_rhs_(t0 + dt, u, f);
-#pragma unroll
-  for (int s = 0; s < NS; ++s)
-    err[s] = f[s] + ((R::C81 * idt) * K(0, s) + (R::C82 * idt) * K(1, s) + (R::C83 * idt) * K(2, s) +
-                     (R::C84 * idt) * K(3, s) + (R::C85 * idt) * K(4, s) + (R::C86 * idt) * K(5, s) +
-                     (R::C87 * idt) * K(6, s));
-  wsolve_(err);
-  st(7, err);
-#pragma unroll
-  for (int s = 0; s < NS; ++s) y1[s] = u[s] + err[s];
+  for (int s = 0; s < NS; ++s) {
+    err[s] = k[s];
+    y1[s] = u[s] + k[s];
+  }
 }
 
 template <int NS>
