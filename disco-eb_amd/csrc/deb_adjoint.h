@@ -874,7 +874,7 @@ __device__ __forceinline__ TD seed_td(double v, double d0) {
 // one forward step from (t0, y0) to y1, its eight stage vectors stored in
 // K[8][NS][64]
 template <int NS>
-__device__ __forceinline__ void step_store(Mode<NS> &m, Ctx &cx, double t0, double h, const double (&y0)[NS],
+__device__ __forceinline__ void step_store(Mode<NS> &m, double t0, double h, const double (&y0)[NS],
                                            double (&y1)[NS], double *K, lds_double *kl) {
   const int lane = lane_id();
   double err[NS];
@@ -882,7 +882,7 @@ __device__ __forceinline__ void step_store(Mode<NS> &m, Ctx &cx, double t0, doub
 #pragma unroll
     for (int s = 0; s < NS; ++s) K[(i * NS + s) * WAVE + lane] = k[s];
   };
-  rodas5_step_s<NS>(m, cx, t0, h, y0, y1, err, store, kl);
+  rodas5_step_s<NS>(m, t0, h, y0, y1, err, store, kl);
 }
 
 // ---------------------------------------------------------------------------
@@ -902,7 +902,7 @@ __device__ __forceinline__ void rodas5_step_vjp(Mode<NS> &m, Ctx &cx, double t0,
   // lane alike)
   __shared__ double cst_[8 * (1 + FT_N)];
   lds_double *const cst = (lds_double *)cst_;
-  factor_call<NS>(m, cx, t0, y0, h);
+  factor_call<NS>(m, t0, y0, h);
   double tw[NS];
   trunc_weights<NS>(m.rd, tw);
   const double it0 = 1.0 / t0;
@@ -1326,6 +1326,7 @@ __device__ __forceinline__ void adjoint_mode(const Params<NS> &P, const AdjArgs 
 #pragma unroll
   for (int s = 0; s < NS; ++s) m.rd[s] = P.rowdesc[s][lane];
   row_consts<NS>(m.rd, cx, m.rk);
+  bg_init(cx, m.bg);
   m.nlev = mode_levels(P.cfg, P.nq);
   const double *tout = P.tau_out + (long long)ci * P.nout;
   const double *dtout = A.dtau + (long long)ci * A.ndir * P.nout;
@@ -1379,6 +1380,7 @@ __device__ __forceinline__ void adjoint_mode(const Params<NS> &P, const AdjArgs 
       mr.pcr = pcr;
       mr.u = (lds_mode_u *)&mu;
       mr.rk = m.rk;
+      mr.bg = m.bg;
       mr.nlev = m.nlev;
       double y[NS], y1[NS];
       const double *yc = chunk_y(chunk);
@@ -1388,7 +1390,7 @@ __device__ __forceinline__ void adjoint_mode(const Params<NS> &P, const AdjArgs 
         double *ry = ring_y(j);
 #pragma unroll
         for (int s = 0; s < NS; ++s) ry[s * WAVE + lane] = y[s];
-        step_store<NS>(mr, cx, tt[j], tt[j + 1] - tt[j], y, y1, ring_k(j), (lds_double *)KBl);
+        step_store<NS>(mr, tt[j], tt[j + 1] - tt[j], y, y1, ring_k(j), (lds_double *)KBl);
 #pragma unroll
         for (int s = 0; s < NS; ++s) y[s] = y1[s];
       }

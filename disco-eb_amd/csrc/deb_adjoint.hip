@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "deb_adjoint.h"
+#include "deb_kargs.h"
 #include "deb_host.h"
 
 namespace deb {
@@ -27,7 +28,8 @@ namespace deb {
 // within a few probes; a wave that finds none after 4 passes gives NaN
 // gradients instead of waiting.  The ring is released when the item is done.
 template <int NS>
-__global__ void __launch_bounds__(WAVE) deb_adjoint_kernel(const Params<NS> P, const AdjArgs A) {
+__global__ void __launch_bounds__(WAVE) deb_adjoint_kernel(const Params<NS> P_, const AdjArgs A) {
+  const Params<NS> &P = kernel_params<NS>();
   // the stage cotangents of one reverse step; between steps the first two
   // [NS][64] blocks stage the output conversion's reverse (output_vjp)
   __shared__ double KBl[7 * NS * WAVE];
@@ -91,7 +93,8 @@ __device__ __forceinline__ void hook_ctx(Ctx &cx, const Params<NS> &P, const Vjp
 }
 
 template <int NS>
-__global__ void __launch_bounds__(WAVE) deb_rhs_vjp_kernel(const Params<NS> P, const VjpHook H) {
+__global__ void __launch_bounds__(WAVE) deb_rhs_vjp_kernel(const Params<NS> P_, const VjpHook H) {
+  const Params<NS> &P = kernel_params<NS>();
   const int item = blockIdx.x;
   if (item >= H.m) return;
   const int lane = lane_id();
@@ -142,7 +145,8 @@ __global__ void __launch_bounds__(WAVE) deb_rhs_vjp_kernel(const Params<NS> P, c
 }
 
 template <int NS>
-__global__ void __launch_bounds__(WAVE) deb_step_vjp_kernel(const Params<NS> P, const VjpHook H) {
+__global__ void __launch_bounds__(WAVE) deb_step_vjp_kernel(const Params<NS> P_, const VjpHook H) {
+  const Params<NS> &P = kernel_params<NS>();
   __shared__ double Kl[8 * NS * WAVE];
   __shared__ double KBl[7 * NS * WAVE];
   __shared__ double pcr[pcr_lds_doubles<NS>()];
@@ -172,7 +176,8 @@ __global__ void __launch_bounds__(WAVE) deb_step_vjp_kernel(const Params<NS> P, 
   double tb = 0.0, hb = 0.0;
   double y1[NS];
   row_consts<NS>(m.rd, cx, m.rk);
-  step_store<NS>(m, cx, t0, h, y, y1, Kl, (lds_double *)KBl);
+  bg_init(cx, m.bg);
+  step_store<NS>(m, t0, h, y, y1, Kl, (lds_double *)KBl);
   rodas5_step_vjp<NS>(m, cx, t0, h, y, yb, thb, tb, hb, Kl, KBl);
   double *yo = H.ybar + (long long)item * P.n;
 #pragma unroll

@@ -302,6 +302,7 @@ __device__ __forceinline__ void integrate_mode(const Params<NS> &P, int ci, int 
 #pragma unroll
   for (int s = 0; s < NS; ++s) m.rd[s] = P.rowdesc[s][lane];
   row_consts<NS>(m.rd, cx, m.rk);
+  bg_init(cx, m.bg);
   m.nlev = mode_levels(P.cfg, P.nq);
   // stage vectors in the kernel's LDS (lds holds fwd_lds_doubles<NS>())
   lds_double *const kl = stage_in_lds<NS>() ? (lds_double *)lds : nullptr;
@@ -347,7 +348,7 @@ __device__ __forceinline__ void integrate_mode(const Params<NS> &P, int ci, int 
       break;
     }
     const double dt = tnext - tprev;
-    rodas5_step<NS>(m, cx, tprev, dt, y, y1, err, kl);
+    rodas5_step<NS>(m, tprev, dt, y, y1, err, kl);
     // filtered, weighted RMS of the scaled error: lanes outside the filter
     // never enter it, so a non-finite unfiltered entry cannot poison it
     const double sc = err[0] / (cf.atol + fmax(fabs(y[0]), fabs(y1[0])) * cf.rtol);
@@ -421,6 +422,7 @@ __device__ __forceinline__ void integrate_batch(const Params<NS> &P, int ci, int
 #pragma unroll
   for (int s = 0; s < NS; ++s) m.rd[s] = P.rowdesc[s][lane];
   row_consts<NS>(m.rd, cx, m.rk);
+  bg_init(cx, m.bg);
   m.nlev = mode_levels(P.cfg, P.nq);
   // stage vectors in the kernel's LDS (lds holds fwd_lds_doubles<NS>())
   lds_double *const kl = stage_in_lds<NS>() ? (lds_double *)lds : nullptr;
@@ -473,7 +475,8 @@ __device__ __forceinline__ void integrate_batch(const Params<NS> &P, int ci, int
 #pragma unroll
       for (int s = 0; s < NS; ++s) y[s] = src[s * WAVE];
       row_consts<NS>(m.rd, cx, m.rk);
-      rodas5_step<NS>(m, cx, tprev, dt, y, y1, err, kl);
+      bg_set_k(m.bg, k);
+      rodas5_step<NS>(m, tprev, dt, y, y1, err, kl);
       // error-norm weights: indices (a, eta, delta_c, delta_b, theta_b, delta_gamma) of slot 0
       double ew = 0.0;
       if (lane == L_A || lane == L_DC || lane == L_DB || lane == L_DG) ew = 1.0;
@@ -543,20 +546,6 @@ __device__ __forceinline__ void integrate_batch(const Params<NS> &P, int ci, int
       if (P.nsteps) P.nsteps[mode0 + b] = steps;
     }
   }
-}
-
-// One workgroup (one wavefront) per (cosmology, k) item; the hardware
-// dispatcher hands the next item to whichever SIMD frees up first, and items
-// are numbered so that the largest k (most steps) start first.
-template <int NS>
-__global__ void __launch_bounds__(WAVE) deb_forward_kernel(const Params<NS> P) {
-  __shared__ double lds[fwd_lds_doubles<NS>()];
-  __shared__ double pcr[pcr_lds_doubles<NS>()];
-  const int item = blockIdx.x;
-  if (item >= P.n_cosmo * P.nk) return;
-  const int ki = P.nk - 1 - item / P.n_cosmo;
-  const int ci = item % P.n_cosmo;
-  integrate_mode<NS>(P, ci, ki, lds, (lds_double *)pcr);
 }
 
 }  // namespace deb

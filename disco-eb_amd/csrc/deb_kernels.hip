@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "deb_forward.h"
+#include "deb_kargs.h"
 #include "deb_host.h"
 
 namespace deb {
@@ -61,10 +62,26 @@ static void *scratch_ptr() {
   return g_scratch_ptr[dev];
 }
 
+// One workgroup (one wavefront) per (cosmology, k) item; the hardware
+// dispatcher hands the next item to whichever SIMD frees up first, and items
+// are numbered so that the largest k (most steps) start first.
+template <int NS>
+__global__ void __launch_bounds__(WAVE) deb_forward_kernel(const Params<NS> P_) {
+  const Params<NS> &P = kernel_params<NS>();
+  __shared__ double lds[fwd_lds_doubles<NS>()];
+  __shared__ double pcr[pcr_lds_doubles<NS>()];
+  const int item = blockIdx.x;
+  if (item >= P.n_cosmo * P.nk) return;
+  const int ki = P.nk - 1 - item / P.n_cosmo;
+  const int ci = item % P.n_cosmo;
+  integrate_mode<NS>(P, ci, ki, lds, (lds_double *)pcr);
+}
+
 // evolve_perturbations_batched: one wavefront per (cosmology, group of B
 // consecutive k), groups of the largest k first.
 template <int NS>
-__global__ void __launch_bounds__(WAVE) deb_forward_batched_kernel(const Params<NS> P, const int B, double *ws) {
+__global__ void __launch_bounds__(WAVE) deb_forward_batched_kernel(const Params<NS> P_, const int B, double *ws) {
+  const Params<NS> &P = kernel_params<NS>();
   __shared__ double lds[fwd_lds_doubles<NS>()];
   __shared__ double pcr[pcr_lds_doubles<NS>()];
   const int ng = P.nk / B;
@@ -78,7 +95,8 @@ __global__ void __launch_bounds__(WAVE) deb_forward_batched_kernel(const Params<
 // The forward solve that also writes every accepted state to the checkpoint
 // tape of the gradient path (deb_solve_forward_tape).
 template <int NS>
-__global__ void __launch_bounds__(WAVE) deb_forward_tape_kernel(const Params<NS> P, const TapeView T) {
+__global__ void __launch_bounds__(WAVE) deb_forward_tape_kernel(const Params<NS> P_, const TapeView T) {
+  const Params<NS> &P = kernel_params<NS>();
   __shared__ double lds[fwd_lds_doubles<NS>()];
   __shared__ double pcr[pcr_lds_doubles<NS>()];
   const int item = blockIdx.x;
@@ -99,7 +117,8 @@ struct HookArgs {
 };
 
 template <int NS>
-__global__ void __launch_bounds__(WAVE) deb_rhs_kernel(const Params<NS> P, const HookArgs<NS> H) {
+__global__ void __launch_bounds__(WAVE) deb_rhs_kernel(const Params<NS> P_, const HookArgs<NS> H) {
+  const Params<NS> &P = kernel_params<NS>();
   const int item = blockIdx.x;
   if (item >= H.m) return;
   const int lane = lane_id();
@@ -115,7 +134,9 @@ __global__ void __launch_bounds__(WAVE) deb_rhs_kernel(const Params<NS> P, const
   }
   RowK<NS> K;
   row_consts<NS>(rd, cx, K);
-  eval_rhs<NS, double>(cx, K, H.t0[item], y, f);
+  BgCache bg;
+  bg_init(cx, bg);
+  eval_rhs<NS>(bg, K, H.t0[item], y, f);
   double *dst = H.y1 + (int64_t)item * P.n;
 #pragma unroll
   for (int s = 0; s < NS; ++s)
@@ -123,7 +144,8 @@ __global__ void __launch_bounds__(WAVE) deb_rhs_kernel(const Params<NS> P, const
 }
 
 template <int NS>
-__global__ void __launch_bounds__(WAVE) deb_step_kernel(const Params<NS> P, const HookArgs<NS> H) {
+__global__ void __launch_bounds__(WAVE) deb_step_kernel(const Params<NS> P_, const HookArgs<NS> H) {
+  const Params<NS> &P = kernel_params<NS>();
   __shared__ double lds[fwd_lds_doubles<NS>()];
   __shared__ double pcr[pcr_lds_doubles<NS>()];
   const int item = blockIdx.x;
@@ -152,8 +174,9 @@ __global__ void __launch_bounds__(WAVE) deb_step_kernel(const Params<NS> P, cons
     y[s] = rd_type(m.rd[s]) != R_NONE ? src[rd_idx(m.rd[s])] : 0.0;
   }
   row_consts<NS>(m.rd, cx, m.rk);
+  bg_init(cx, m.bg);
   const double t0 = H.t0[item];
-  rodas5_step<NS>(m, cx, t0, H.t1[item] - t0, y, y1, err, stage_in_lds<NS>() ? (lds_double *)lds : nullptr);
+  rodas5_step<NS>(m, t0, H.t1[item] - t0, y, y1, err, stage_in_lds<NS>() ? (lds_double *)lds : nullptr);
   double *d1 = H.y1 + (int64_t)item * P.n;
   double *de = H.err + (int64_t)item * P.n;
 #pragma unroll
@@ -166,7 +189,8 @@ __global__ void __launch_bounds__(WAVE) deb_step_kernel(const Params<NS> P, cons
 
 // test hook: the start time of every (cosmology, k) mode
 // (determine_starting_time and 0.99 min(min tau_out, tau*))
-__global__ void __launch_bounds__(WAVE) deb_start_kernel(const Params<1> P, double *ts) {
+__global__ void __launch_bounds__(WAVE) deb_start_kernel(const Params<1> P_, double *ts) {
+  const Params<1> &P = kernel_params<1>();
   const int item = blockIdx.x;
   if (item >= P.n_cosmo * P.nk) return;
   const int ci = item / P.nk;

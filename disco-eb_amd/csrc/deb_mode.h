@@ -643,6 +643,196 @@ __device__ __forceinline__ void row_consts(const uint32_t (&rd)[NS], const Ctx &
   }
 }
 
+// 1/x and component-wise selection in plain doubles and along a
+__device__ __forceinline__ double rcp_a(double x) { return rcp_nr(x); }
+__device__ __forceinline__ dual rcp_a(dual x) {
+  const double r = rcp_nr(x.v);
+  return {r, -(r * r) * x.d};
+}
+__device__ __forceinline__ double sel(bool c, double x, double y) { return c ? x : y; }
+__device__ __forceinline__ dual sel(bool c, dual x, dual y) { return {c ? x.v : y.v, c ? x.d : y.d}; }
+
+// log x for positive normal x, NaN otherwise: x = m 2^e with m in
+// [1/sqrt 2, sqrt 2], log m = 2 atanh z, z = (m - 1) / (m + 1), |z| < 0.172,
+// by its series up to z^23 (remainder below 1e-19); about one ulp of log x
+// where e != 0, 2e-16 absolute elsewhere.  A third of the instructions of the
+// library's log, which carries the result to less than an ulp.
+__device__ __forceinline__ double log_pos(double x) {
+  const int hi = __double2hiint(x);
+  int e = (hi >> 20) - 1023;
+  double m = __hiloint2double((hi & 0xfffff) | 0x3ff00000, __double2loint(x));
+  const bool up = m > 1.4142135623730951;
+  m = up ? 0.5 * m : m;
+  e = up ? e + 1 : e;
+  const double z = (m - 1.0) * rcp_nr(m + 1.0), w = z * z;
+  double p = 2.0 / 23.0;
+  p = fma(p, w, 2.0 / 21.0);
+  p = fma(p, w, 2.0 / 19.0);
+  p = fma(p, w, 2.0 / 17.0);
+  p = fma(p, w, 2.0 / 15.0);
+  p = fma(p, w, 2.0 / 13.0);
+  p = fma(p, w, 2.0 / 11.0);
+  p = fma(p, w, 2.0 / 9.0);
+  p = fma(p, w, 2.0 / 7.0);
+  p = fma(p, w, 2.0 / 5.0);
+  p = fma(p, w, 2.0 / 3.0);
+  const double d = (double)e;
+  // ln 2 in two parts, the first exact in products with e
+  const double r = fma(d, 6.93147180369123816490e-01, fma(2.0, z, fma(z * w, p, d * 1.90821492927058770002e-10)));
+  return x >= 2.2250738585072014e-308 && x <= 1.7976931348623157e308 ? r : __builtin_nan("");
+}
+
+// ---------------------------------------------------------------------------
+// The background of one mode's right-hand sides.  The cosmology's numbers are
+// combined once per mode.  The three splines' knots live in registers, one
+// interval per lane: lane 4 w + j holds interval base_j + w of spline j, so
+// sixteen consecutive intervals of each are at hand, a ballot finds the lanes
+// whose interval holds log a, and memory is read only when log a leaves a
+// window (from six knots per right-hand side through the caches before).
+struct BgCache {
+  const double *x;  // the lane's spline: knots x, then y, then S, n each
+  int n;
+  double xlo, xhi;  // the lane's interval, the first and the last one open to infinity
+  double x0, ih, y0, y1, s0, s1;  // its knots: 1/h, S h^2 / 6
+  double gm, ggr, gn, gde, gk;    // densities: grhom Omega_m, grhog + grhor Neff, grhor Nmnu, grhom Omega_DE, grhom Omega_k
+  double w0, wa, e1;              // e1 = -3 (1 + w0 + wa)
+  double kth, pb;                 // opacity / x_e a^2; (4/3) rho_g / rho_b a
+  double cs2Q, k2, ik2;
+  bool lambda;
+};
+
+__device__ __forceinline__ void bg_set_k(BgCache &g, double k) {
+  g.k2 = k * k;
+  g.ik2 = 1.0 / g.k2;
+}
+
+__device__ __forceinline__ void bg_init(const Ctx &cx, BgCache &g) {
+  const deb_cosmo_t &c = *cx.c;
+  const int j = lane_id() & 3;
+  const Spl s0 = cx.sp[DEB_SPL_CS2A_LOGA], s1 = cx.sp[DEB_SPL_XE_LOGA], s2 = cx.sp[DEB_SPL_LOGRHONU_LOGA];
+  g.x = j == 0 ? s0.x : (j == 1 ? s1.x : s2.x);
+  g.n = j == 0 ? s0.n : (j == 1 ? s1.n : s2.n);
+  g.xlo = INFINITY;  // no interval yet
+  g.xhi = g.x0 = g.ih = g.y0 = g.y1 = g.s0 = g.s1 = 0.0;
+  g.gm = c.grhom * c.Omegam;
+  g.ggr = c.grhog + c.grhor * c.Neff;
+  g.gn = c.grhor * c.Nmnu;
+  g.gde = c.grhom * c.OmegaDE;
+  g.gk = c.grhom * c.Omegak;
+  g.w0 = c.w_DE_0;
+  g.wa = c.w_DE_a;
+  g.e1 = -3.0 * (1.0 + c.w_DE_0 + c.w_DE_a);
+  g.kth = 2.3038921003709498e-9 * (1.0 - c.YHe) * c.Omegab * c.H0 * c.H0;
+  g.pb = (4.0 / 3.0) * (c.grhog / (c.grhom * c.Omegab));
+  g.cs2Q = c.cs2_DE;
+  g.lambda = cx.lambda;
+  bg_set_k(g, cx.k);
+}
+
+// moves every spline's window so that it holds the interval of v (the rule of
+// spl_interval), three intervals behind it and twelve ahead; returns the lane
+// that holds the interval of the lane's own spline
+__device__ __forceinline__ int bg_seek(BgCache &g, double v) {
+  const double *x = g.x, *y = g.x + g.n, *S = y + g.n;
+  int lo = 0, hi = g.n;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (x[mid] < v) lo = mid + 1; else hi = mid;
+  }
+  int i = lo - 1;
+  i = i < 0 ? 0 : (i > g.n - 2 ? g.n - 2 : i);
+  const int base = i < 3 ? 0 : i - 3;
+  const int own = base + (lane_id() >> 2);
+  const int c = own > g.n - 2 ? g.n - 2 : own;
+  const double x0 = x[c], x1 = x[c + 1], h = x1 - x0, h26 = h * h / 6.0;
+  g.x0 = x0;
+  g.ih = 1.0 / h;
+  g.y0 = y[c];
+  g.y1 = y[c + 1];
+  g.s0 = S[c] * h26;
+  g.s1 = S[c + 1] * h26;
+  g.xlo = own > g.n - 2 ? INFINITY : (own == 0 ? -INFINITY : x0);
+  g.xhi = own == g.n - 2 ? INFINITY : x1;
+  return (i - base) * 4 + (lane_id() & 3);
+}
+
+// background quantities at a, as far as the rows need them
+template <typename T>
+struct BgRow {
+  T a, aH, iaH, ia, ia2, opac, cs2, po, rhoQ;
+};
+
+// the spline's value at v in units of its interval, and along log a
+__device__ __forceinline__ double bg_piece(const BgCache &g, double v) {
+  const double B = (v - g.x0) * g.ih, A = 1.0 - B;
+  return A * g.y0 + B * g.y1 + ((A * A * A - A) * g.s0 + (B * B * B - B) * g.s1);
+}
+__device__ __forceinline__ double bg_slope(const BgCache &g, double v) {
+  const double B = (v - g.x0) * g.ih, A = 1.0 - B;
+  return (g.y1 - g.y0 + ((3.0 * B * B - 1.0) * g.s1 - (3.0 * A * A - 1.0) * g.s0)) * g.ih;
+}
+
+template <typename T>
+__device__ __forceinline__ BgRow<T> background_row(BgCache &g, T a) {
+  constexpr bool D = !std::is_same<T, double>::value;
+  const int lane = lane_id();
+  const double av = vval(a);
+  const double loga = log_pos(av);
+  const uint64_t in = __ballot(g.xlo < loga && loga <= g.xhi);
+  const uint64_t m0 = in & 0x1111111111111111ull, m1 = in & 0x2222222222222222ull, m2 = in & 0x4444444444444444ull;
+  int l0, l1, l2;
+  if (m0 != 0 && m1 != 0 && m2 != 0) {
+    l0 = __builtin_ctzll(m0);
+    l1 = __builtin_ctzll(m1);
+    l2 = __builtin_ctzll(m2);
+  } else {
+    const int l = bg_seek(g, loga);
+    l0 = __builtin_amdgcn_readlane(l, 0);
+    l1 = __builtin_amdgcn_readlane(l, 1);
+    l2 = __builtin_amdgcn_readlane(l, 2);
+  }
+  const double val = bg_piece(g, loga);
+  // both exponentials at once: lane 0 that of log rho_nu, the others dark energy's
+  const double lrnu = readlane(val, l2);
+  const double ex = exp(lane == 0 ? lrnu : g.e1 * loga + 3.0 * (av - 1.0) * g.wa);
+  BgRow<T> b;
+  T cs2a, xe, rhonu;
+  b.a = a;
+  b.ia = rcp_a(a);
+  if constexpr (D) {
+    const double slope = bg_slope(g, loga);
+    const double ia = b.ia.v;
+    const double e0 = readlane(ex, 0), e1 = readlane(ex, 1);
+    cs2a = T{readlane(val, l0), readlane(slope, l0) * ia};
+    xe = T{readlane(val, l1), readlane(slope, l1) * ia};
+    rhonu = T{e0, e0 * (readlane(slope, l2) * ia)};
+    b.rhoQ = T{e1, e1 * (g.e1 * ia + 3.0 * g.wa)};
+  } else {
+    cs2a = readlane(val, l0);
+    xe = readlane(val, l1);
+    rhonu = readlane(ex, 0);
+    b.rhoQ = readlane(ex, 1);
+  }
+  b.ia2 = b.ia * b.ia;
+  b.cs2 = cs2a * b.ia;
+  b.opac = g.kth * xe * b.ia2;
+  b.po = (g.pb * b.ia) * b.opac;
+  const T grho3 = (g.gm * b.ia + (g.ggr + g.gn * rhonu) * b.ia2 + g.gde * b.rhoQ * (a * a) + g.gk) * (1.0 / 3.0);
+  // aH = sqrt(grho3) and its reciprocal from one estimate, the root corrected by its residual
+  const double r = rsq_nr(vval(grho3));
+  double h = vval(grho3) * r;
+  h = fma(fma(-h, h, vval(grho3)), 0.5 * r, h);
+  if constexpr (D) {
+    const double hd = 0.5 * grho3.d * r;
+    b.aH = T{h, hd};
+    b.iaH = T{r, -hd * (r * r)};
+  } else {
+    b.aH = h;
+    b.iaH = r;
+  }
+  return b;
+}
+
 // v_q = (1 + x^2)^(-1/2) and 1/v_q of x = a m_nu / q
 __device__ __forceinline__ void bin_velocity(double a, double aq, double &vq, double &ivq) {
   const double x = a * aq, s2 = 1.0 + x * x;
@@ -659,7 +849,8 @@ __device__ __forceinline__ void bin_velocity(dual a, double aq, dual &vq, dual &
 
 // the coefficients of slot s's rows at background b, from their constants
 template <int NS, typename T>
-__device__ __forceinline__ Coef<T> row_lin(const RowK<NS> &K, int s, const Bg<T> &b, const Ctx &cx, double invtau) {
+__device__ __forceinline__ Coef<T> row_lin(const RowK<NS> &K, int s, const BgRow<T> &b, const BgCache &g,
+                                           double invtau) {
   Coef<T> r;
   T vq = tconst<T>(1.0), ivq = tconst<T>(1.0);
   if ((K.qmask >> s) & 1u) bin_velocity(b.a, K.aq[s], vq, ivq);
@@ -671,39 +862,36 @@ __device__ __forceinline__ Coef<T> row_lin(const RowK<NS> &K, int s, const Bg<T>
   r.upi = K.upi[s] * b.opac;
   r.cpi = tconst<T>(K.cpi[s]);
   r.leaf = tconst<T>(0.0);
-  const T gh = b.ia2 * b.iaH;
-  r.ch = K.ch[s] * (ivq * gh);
+  r.ch = K.ch[s] * (ivq * (b.ia2 * b.iaH));
   r.ceta = K.ceta[s] * b.ia2;
   r.c1 = (-K.ch[s]) * ((ivq + vq) * b.ia);
   if (s == 0) {
     const int lane = lane_id();
-    const double k2 = cx.k * cx.k;
-    const bool dcb = lane == L_DC || lane == L_DB, eta = lane == L_ETA, tb = lane == L_TB, tg = lane == L_TG;
-    const T po = b.pb43 * b.opac;
+    const bool dcb = (lane == L_DC) | (lane == L_DB), eta = lane == L_ETA, tb = lane == L_TB, tg = lane == L_TG;
     r.leaf = tconst<T>(K.leaf);
     r.diag = r.diag - K.dah * b.aH;
-    r.diag = tb ? r.diag - po : r.diag;
-    r.sub = tb ? k2 * b.cs2 : (tg ? b.opac : r.sub);
-    r.sup = tb ? po : r.sup;
-    r.ch = (dcb || eta) ? K.ch[0] * (eta ? b.iaH : b.ia * b.iaH) : r.ch;
-    r.c1 = (dcb || eta) ? tconst<T>(eta ? 0.0 : -K.ch[0]) : r.c1;
-    r.ceta = (tb || lane == L_TC) ? K.ceta[0] * b.ia : r.ceta;
+    r.diag = sel(tb, r.diag - b.po, r.diag);
+    r.sub = sel(tb, g.k2 * b.cs2, sel(tg, b.opac, r.sub));
+    r.sup = sel(tb, b.po, r.sup);
+    r.ch = sel(dcb, K.ch[0] * (b.ia * b.iaH), sel(eta, K.ch[0] * b.iaH, r.ch));
+    r.c1 = sel(dcb | eta, tconst<T>(eta ? 0.0 : -K.ch[0]), r.c1);
+    r.ceta = sel(tb | (lane == L_TC), K.ceta[0] * b.ia, r.ceta);
     // dark-energy fluid (frozen for a cosmological constant)
-    if (!cx.lambda) {
-      const double cs2Q = cx.c->cs2_DE, gde = cx.c->grhom * cx.c->OmegaDE;
-      const double ik2 = 1.0 / k2;
-      const T opw = 1.0 + b.w;
-      const T rq = gde * b.rhoQ * (b.a * b.a);
+    if (!g.lambda) {
       const bool dq = lane == L_DQ, tq = lane == L_TQ;
-      const T dc = cs2Q - b.ca2;
-      r.diag = dq ? -3.0 * (cs2Q - b.w) * b.aH : r.diag;
-      r.sup = dq ? -opw - 9.0 * opw * dc * b.aH * b.aH * ik2 : r.sup;
-      r.uh = dq ? -0.5 * opw : r.uh;
-      r.ch = dq ? rq * b.iaH : r.ch;
-      r.sub = tq ? cs2Q / opw * k2 : r.sub;
-      r.ceta = tq ? opw * rq * (0.5 * ik2) : r.ceta;
-      const T q1 = rq + 3.0 * cs2Q * rq, q2 = 3.0 * dc * (3.0 * b.aH * ik2) * opw * rq;
-      r.c1 = (dq || tq) ? -b.a * (dq ? q1 : q2) : r.c1;
+      const T w = g.w0 + g.wa * (1.0 - b.a);
+      const T opw = 1.0 + w;
+      const T dc = g.cs2Q - w - (g.wa * (1.0 / 3.0)) * (b.a * rcp_a(opw + 1e-6));  // c_s^2 - c_a^2
+      const T rq = g.gde * b.rhoQ * (b.a * b.a);
+      const T oaH = opw * b.aH * dc;
+      r.diag = sel(dq, -3.0 * (g.cs2Q - w) * b.aH, r.diag);
+      r.sup = sel(dq, -opw - (9.0 * g.ik2) * (oaH * b.aH), r.sup);
+      r.uh = sel(dq, -0.5 * opw, r.uh);
+      r.ch = sel(dq, rq * b.iaH, r.ch);
+      r.sub = sel(tq, (g.cs2Q * g.k2) * rcp_a(opw), r.sub);
+      r.ceta = sel(tq, (0.5 * g.ik2) * (opw * rq), r.ceta);
+      const T arq = b.a * rq;
+      r.c1 = sel(dq, (-(1.0 + 3.0 * g.cs2Q)) * arq, sel(tq, (-9.0 * g.ik2) * (oaH * arq), r.c1));
     }
   }
   return r;

@@ -29,6 +29,7 @@ template <int NS>
 struct Mode {
   uint32_t rd[NS];
   RowK<NS> rk;       // the rows' constants (row_consts)
+  BgCache bg;        // the background's constants and spline windows (bg_init)
   // PCR factors of W_B: d' = sig*d + al*d[i-s] + be*d[i+s] at level s = 2^L;
   // al and be live in the wave's LDS ([PCR_LEVELS][2][NS][64], pcr_lds_doubles)
   lds_double *pcr;
@@ -49,19 +50,18 @@ struct Mode {
   int nlev;
 };
 
-// evaluate f (T-valued) at (tau, y); optionally return the coefficient rows
+// evaluate f (T-valued) at (tau, y) and the coefficient rows cf
 template <int NS, typename T>
-__device__ __forceinline__ void eval_rhs(Ctx &cx, const RowK<NS> &K, double tau, const double (&y)[NS],
-                                         T (&f)[NS], Coef<T> (*co)[NS] = nullptr, T *aH_out = nullptr) {
+__device__ __forceinline__ void eval_rhs(BgCache &bg, const RowK<NS> &K, double tau, const double (&y)[NS],
+                                         T (&f)[NS], Coef<T> (&cf)[NS]) {
   const int lane = lane_id();
   double a0 = readlane(y[0], L_A);
   T a;
   if constexpr (sizeof(T) == sizeof(double)) a = a0; else a = T{a0, 1.0};
-  Bg<T> b = background<T>(cx, a);
-  const double invtau = 1.0 / tau;
-  Coef<T> cf[NS];
+  const BgRow<T> b = background_row(bg, a);
+  const double invtau = rcp_nr(tau);
 #pragma unroll
-  for (int s = 0; s < NS; ++s) cf[s] = row_lin<NS, T>(K, s, b, cx, invtau);
+  for (int s = 0; s < NS; ++s) cf[s] = row_lin<NS, T>(K, s, b, bg, invtau);
   // functionals h', eta', Pi, f_1
   constexpr int NV = (sizeof(T) == sizeof(double)) ? 4 : 8;
   double part[NV];
@@ -108,11 +108,12 @@ __device__ __forceinline__ void eval_rhs(Ctx &cx, const RowK<NS> &K, double tau,
     }
     f[s] = v;
   }
-  if (co) {
-#pragma unroll
-    for (int s = 0; s < NS; ++s) (*co)[s] = cf[s];
-  }
-  if (aH_out) *aH_out = b.aH;
+}
+template <int NS>
+__device__ __forceinline__ void eval_rhs(BgCache &bg, const RowK<NS> &K, double tau, const double (&y)[NS],
+                                         double (&f)[NS]) {
+  Coef<double> cf[NS];
+  eval_rhs<NS, double>(bg, K, tau, y, f, cf);
 }
 
 // df/dtau: only the hierarchy truncation rows depend on tau explicitly
@@ -157,13 +158,13 @@ __device__ __forceinline__ void bsolve(const Mode<NS> &m, double (&x)[NS]) {
 
 // factorisation of W at (tau0, y0) for step size h; f0 = f(tau0, y0)
 template <int NS>
-__device__ __forceinline__ void factor(Mode<NS> &m, Ctx &cx, double tau0, const double (&y0)[NS], double h,
+__device__ __forceinline__ void factor(Mode<NS> &m, double tau0, const double (&y0)[NS], double h,
                                        double (&f0)[NS]) {
   const int lane = lane_id();
   constexpr double gamma = 0.19;
   dual fd[NS];
   Coef<dual> co[NS];
-  eval_rhs<NS, dual>(cx, m.rk, tau0, y0, fd, &co);
+  eval_rhs<NS, dual>(m.bg, m.rk, tau0, y0, fd, co);
 #pragma unroll
   for (int s = 0; s < NS; ++s) f0[s] = fd[s].v;
   m.u->gh = gamma * h;
@@ -346,9 +347,9 @@ struct R5 {
 // Out-of-line factorisation, for the reverse of a step (next to much other
 // live state): as a call, the step factors stay in memory instead of registers.
 template <int NS>
-__device__ __noinline__ void factor_call(Mode<NS> &m, Ctx &cx, double tau0, const double (&y0)[NS], double h) {
+__device__ __noinline__ void factor_call(Mode<NS> &m, double tau0, const double (&y0)[NS], double h) {
   double f0[NS];
-  factor<NS>(m, cx, tau0, y0, h, f0);
+  factor<NS>(m, tau0, y0, h, f0);
 }
 
 // Rodas5 tableau in flattened form (constant memory, read with wave-uniform
@@ -384,12 +385,12 @@ __constant__ double kd[8] = {R5::d1, R5::d2, R5::d3, R5::d4, R5::d5, 0.0, 0.0, 0
 // 7 x NS x 64 doubles) the stage vectors k1..k7 are kept there, else in
 // registers.
 template <int NS, class Store>
-__device__ __forceinline__ void rodas5_step_s(Mode<NS> &m, Ctx &cx, double t0, double dt, const double (&y0)[NS],
+__device__ __forceinline__ void rodas5_step_s(Mode<NS> &m, double t0, double dt, const double (&y0)[NS],
                                               double (&y1)[NS], double (&err)[NS], Store st,
                                               lds_double *kl = nullptr) {
   const int lane = lane_id();
   double k[NS], u[NS], f[NS], dT[NS];
-  factor<NS>(m, cx, t0, y0, dt, f);
+  factor<NS>(m, t0, y0, dt, f);
   dfdtau<NS>(m.rk, t0, y0, dT);
   // the stage vectors start from zero: a stage then sums over fixed columns of
   // the tableau (zero from column i on) without meeting what an earlier step,
@@ -420,31 +421,28 @@ __device__ __forceinline__ void rodas5_step_s(Mode<NS> &m, Ctx &cx, double t0, d
 #pragma unroll
       for (int s = 0; s < NS; ++s) du[s] = i >= 6 ? u[s] + k[s] : y0[s];
       const double la = i >= 6 ? 0.0 : 1.0;
+      auto add = [&](auto first, auto count) {
+        constexpr int J0 = decltype(first)::value, NJ = decltype(count)::value;
+        double kj[NJ][NS];
 #pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const double aij = la * kA[i][j], cij = kC[i][j];
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
-        for (int s = 0; s < NS; ++s) {
-          const double kj = K(j, s);
-          du[s] += aij * kj;
-          ck[s] += cij * kj;
-        }
-      }
-      if (i > 3) {
+          for (int s = 0; s < NS; ++s) kj[j][s] = K(J0 + j, s);
 #pragma unroll
-        for (int j = 3; j < 7; ++j) {
-          const double aij = la * kA[i][j], cij = kC[i][j];
+        for (int j = 0; j < NJ; ++j) {
+          const double aij = la * kA[i][J0 + j], cij = kC[i][J0 + j];
 #pragma unroll
           for (int s = 0; s < NS; ++s) {
-            const double kj = K(j, s);
-            if (j < 5) du[s] += aij * kj;
-            ck[s] += cij * kj;
+            if (J0 + j < 5) du[s] += aij * kj[j][s];
+            ck[s] += cij * kj[j][s];
           }
         }
-      }
+      };
+      add(std::integral_constant<int, 0>{}, std::integral_constant<int, 3>{});
+      if (i > 3) add(std::integral_constant<int, 3>{}, std::integral_constant<int, 4>{});
 #pragma unroll
       for (int s = 0; s < NS; ++s) u[s] = du[s];
-      eval_rhs<NS, double>(cx, m.rk, t0 + kc[i] * dt, u, f);
+      eval_rhs<NS>(m.bg, m.rk, t0 + kc[i] * dt, u, f);
     }
     const double hd = dt * kd[i];
 #pragma unroll
@@ -473,9 +471,9 @@ __device__ __forceinline__ void rodas5_step_s(Mode<NS> &m, Ctx &cx, double t0, d
 }
 
 template <int NS>
-__device__ __forceinline__ void rodas5_step(Mode<NS> &m, Ctx &cx, double t0, double dt, const double (&y0)[NS],
+__device__ __forceinline__ void rodas5_step(Mode<NS> &m, double t0, double dt, const double (&y0)[NS],
                                             double (&y1)[NS], double (&err)[NS], lds_double *kl = nullptr) {
-  rodas5_step_s<NS>(m, cx, t0, dt, y0, y1, err, [](int, const double (&)[NS]) {}, kl);
+  rodas5_step_s<NS>(m, t0, dt, y0, y1, err, [](int, const double (&)[NS]) {}, kl);
 }
 
 }  // namespace deb
