@@ -33,6 +33,12 @@ using TD = dn<1 + MAXDIR>;          // (a or tau, theta_1..theta_MAXDIR)
 // device-assembly test of the build checks this for every outlined function.
 #define DEB_OUTLINE __device__ __noinline__
 
+__device__ __forceinline__ void lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
 // ---------------------------------------------------------------------------
 // cross-lane moves and reductions of composite scalars, component by
 // component (member access only)
@@ -223,6 +229,61 @@ __device__ __forceinline__ void features_t(Ctx &cx, T a, T (&F)[FT_N]) {
   features_of<T>(cx, a, b, F);
 }
 
+// the features from the right-hand side's background (background_row), in
+// plain doubles or along a
+template <class T>
+__device__ __forceinline__ void features_row(const Ctx &cx, const BgCache &g, const BgRow<T> &b, T (&F)[FT_N]) {
+  const deb_cosmo_t &c = *cx.c;
+  const T w = g.w0 + g.wa * (1.0 - b.a);
+  F[FT_A] = b.a;
+  F[FT_AH] = b.aH;
+  F[FT_IAH] = b.iaH;
+  F[FT_OPAC] = b.opac;
+  F[FT_CS2] = b.cs2;
+  F[FT_PB43] = g.pb * b.ia;
+  F[FT_RC] = (c.grhom * (c.Omegam - c.Omegab)) * b.ia;
+  F[FT_RB] = (c.grhom * c.Omegab) * b.ia;
+  F[FT_RG] = c.grhog * b.ia2;
+  F[FT_RR] = (c.grhor * c.Neff) * b.ia2;
+  F[FT_RN] = g.gn * b.ia2;
+  F[FT_RQ] = g.gde * b.rhoQ * (b.a * b.a);
+  F[FT_W] = w;
+  F[FT_CA2] = w + (g.wa * (1.0 / 3.0)) * (b.a * rcp_a(1.0 + w + 1e-6));
+  F[FT_CS2Q] = tconst<T>(g.cs2Q);
+  F[FT_AMNU] = tconst<T>(c.amnu);
+}
+
+// the mode's background at a; the spline windows go back to memory only when
+// they have moved
+template <int NS, class T>
+__device__ __forceinline__ BgRow<T> mode_background(Mode<NS> &m, BgCache &g, T a) {
+  g = m.bg;
+  const double lo = g.xlo, hi = g.xhi;
+  const BgRow<T> b = background_row(g, a);
+  if (__ballot(!(lo == g.xlo && hi == g.xhi)) != 0) m.bg = g;
+  return b;
+}
+
+// The 16 sums over the wave of v, one per lane: lane l returns that of
+// v[l & 15].  The butterfly of wave_sum with the values split between the
+// partners at each of the row's four exchanges: 111 instructions, where 16
+// whole sums take 288.
+__device__ __forceinline__ double wave_sum_spread(const double (&v)[16]) {
+  const int lane = lane_id();
+  const bool b3 = (lane & 8) != 0, b2 = (lane & 4) != 0, b1 = (lane & 2) != 0, b0 = (lane & 1) != 0;
+  double w[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) w[i] = (b3 ? v[i + 8] : v[i]) + row_partner<3>(b3 ? v[i] : v[i + 8]);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = (b2 ? w[i + 4] : w[i]) + row_partner<2>(b2 ? w[i] : w[i + 4]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) w[i] = (b1 ? w[i + 2] : w[i]) + row_partner<1>(b1 ? w[i] : w[i + 2]);
+  double r = (b0 ? w[1] : w[0]) + row_partner<0>(b0 ? w[0] : w[1]);
+  r += from_lane(r, lane ^ 16);
+  r += from_lane(r, lane ^ 32);
+  return r;
+}
+
 // Values of the functionals of Y and of the "where they enter" sums of w that
 // the first-order contraction below needs, plus (optionally) the transposed
 // right-hand side A(a)^T w -- one plain-double pass over the rows.
@@ -233,40 +294,17 @@ struct RowSumsT {
 };
 using RowSums = RowSumsT<double>;
 
-// With DFA, also the features' derivatives along a (dfa_out), from a dual
-// evaluation beside the plain one (the plain values feed the rows unchanged).
-template <int NS, bool TAPPLY, bool DFA = false>
-__device__ __forceinline__ RowSums coef_pass_body(Ctx &cx, const uint32_t (&rd)[NS], double a, double invtau,
-                                                  const double (&w_in)[NS], const double (&Y_in)[NS],
-                                                  double (&out)[NS], double (&fv_out)[FT_N],
-                                                  double *dfa_out = nullptr) {
+template <int NS>
+__device__ __forceinline__ RowSums coef_pass_body(const RowK<NS> &K, const BgCache &g, const BgRow<double> &b,
+                                                  double invtau, const double (&w)[NS], const double (&Y)[NS],
+                                                  double (&out)[NS]) {
   const int lane = lane_id();
-  double w[NS], Y[NS];
-#pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    w[s] = w_in[s];
-    Y[s] = Y_in[s];
-  }
-  const Bg<double> b = background<double>(cx, a);
-  double fv[FT_N];
-  features_of<double>(cx, a, b, fv);
-#pragma unroll
-  for (int m = 0; m < FT_N; ++m) fv_out[m] = fv[m];
-  if constexpr (DFA) {
-    dual ad;
-    ad.v = a;
-    ad.d = 1.0;
-    dual Fd[FT_N];
-    features_t<dual>(cx, ad, Fd);
-#pragma unroll
-    for (int m = 0; m < FT_N; ++m) dfa_out[m] = Fd[m].d;
-  }
   double o[NS];
   double part[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   double cc[4][NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    Coef<double> r = row_coef_slot<double>(rd[s], b, cx, invtau, s == 0);
+    const Coef<double> r = row_lin<NS, double>(K, s, b, g, invtau);
     part[0] += r.ch * Y[s];
     part[1] += r.ceta * Y[s];
     part[2] += r.cpi * Y[s];
@@ -274,34 +312,45 @@ __device__ __forceinline__ RowSums coef_pass_body(Ctx &cx, const uint32_t (&rd)[
     part[4] += r.uh * w[s];
     part[5] += r.ueta * w[s];
     part[6] += r.upi * w[s];
-    if constexpr (TAPPLY) {
-      o[s] = r.diag * w[s] + from_next(r.sub * w[s]) + from_prev(r.sup * w[s]);
-      if (s == 0) {
-        const double lw = r.leaf * w[0];
-        const double l_dg = readlane(lw, L_DG), l_tg = readlane(lw, L_TG);
-        if (lane == L_TG) o[0] += l_dg;
-        if (lane == L_DG) o[0] += l_tg;
-      }
-      cc[0][s] = r.ch;
-      cc[1][s] = r.ceta;
-      cc[2][s] = r.cpi;
-      cc[3][s] = r.c1;
+    o[s] = r.diag * w[s] + from_next(r.sub * w[s]) + from_prev(r.sup * w[s]);
+    if (s == 0) {
+      const double lw = r.leaf * w[0];
+      const double l_dg = readlane(lw, L_DG), l_tg = readlane(lw, L_TG);
+      if (lane == L_TG) o[0] += l_dg;
+      if (lane == L_DG) o[0] += l_tg;
     }
+    cc[0][s] = r.ch;
+    cc[1][s] = r.ceta;
+    cc[2][s] = r.cpi;
+    cc[3][s] = r.c1;
   }
   wave_sum<7>(part);
   RowSums rs{part[0], part[1], part[2], part[3], part[4], part[5], part[6]};
-  if constexpr (TAPPLY) {
-    const double wahp = readlane(w[0], L_AHP);
+  const double wahp = readlane(w[0], L_AHP);
 #pragma unroll
-    for (int s = 0; s < NS; ++s) out[s] = o[s] + cc[0][s] * rs.sh + cc[1][s] * rs.se + cc[2][s] * rs.sp + cc[3][s] * wahp;
-  }
+  for (int s = 0; s < NS; ++s) out[s] = o[s] + cc[0][s] * rs.sh + cc[1][s] * rs.se + cc[2][s] * rs.sp + cc[3][s] * wahp;
   return rs;
 }
-template <int NS, bool TAPPLY, bool DFA = false>
-DEB_OUTLINE RowSums coef_pass(Ctx &cx, const uint32_t (&rd)[NS], double a, double invtau,
-                              const double (&w_in)[NS], const double (&Y_in)[NS], double (&out)[NS],
-                              double (&fv_out)[FT_N], double *dfa_out = nullptr) {
-  return coef_pass_body<NS, TAPPLY, DFA>(cx, rd, a, invtau, w_in, Y_in, out, fv_out, dfa_out);
+// the same as a call, with the features at a (the operator's test hook)
+template <int NS>
+DEB_OUTLINE RowSums coef_pass(Mode<NS> &m, Ctx &cx, double a, double invtau, const double (&w_in)[NS],
+                              const double (&Y_in)[NS], double (&out)[NS], double (&fv_out)[FT_N]) {
+  const RowK<NS> K = m.rk;
+  BgCache g;
+  double w[NS], Y[NS], o[NS], F[FT_N];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    w[s] = w_in[s];
+    Y[s] = Y_in[s];
+  }
+  const BgRow<double> b = mode_background<NS>(m, g, a);
+  const RowSums rs = coef_pass_body<NS>(K, g, b, invtau, w, Y, o);
+  features_row(cx, g, b, F);
+#pragma unroll
+  for (int s = 0; s < NS; ++s) out[s] = o[s];
+#pragma unroll
+  for (int q = 0; q < FT_N; ++q) fv_out[q] = F[q];
+  return rs;
 }
 
 // Partials of the rows' sum_fields mul[q][f] coef_f with respect to the
@@ -587,39 +636,6 @@ DEB_OUTLINE void feature_partials(const Ctx &cx, const uint32_t (&rd)[NS], const
   feature_partials_body<NS, K, T>(cx, rd, fv_in, Y_in, w_in, rs_in, fb);
 }
 
-// The feature partials of one reverse stage at five slots (after its row pass
-// and row sums): both contractions summed over the wave, the stage's (at its
-// features fv) stored to fb_out and contracted with the features'
-// a-derivatives dfa into the returned a-direction of the stage cotangent, the
-// J-term's (at the features fvJ of a0) accumulated into fbJ.  fvJ, fbJ and
-// fb_out: one copy per wave in LDS.
-template <int NS>
-DEB_OUTLINE double stage_partials(const Ctx &cx, const uint32_t (&rd)[NS], const double (&fv_in)[FT_N],
-                                  const lds_double *fvJ_in, const double (&dfa_in)[FT_N],
-                                  const double (&Y_in)[2][NS], const double (&w_in)[2][NS],
-                                  const RowSums (&rs_in)[2], lds_double *fbJ_io, lds_double *fb_out) {
-  double fvs[2][FT_N], fbs[2][FT_N];
-#pragma unroll
-  for (int q = 0; q < FT_N; ++q) {
-    fvs[0][q] = fv_in[q];
-    fvs[1][q] = (double)fvJ_in[q];
-    fbs[0][q] = 0.0;
-    fbs[1][q] = 0.0;
-  }
-  feature_partials_body<NS, 2>(cx, rd, fvs, Y_in, w_in, rs_in, fbs);
-  wave_sum<FT_N>(fbs[0]);
-  wave_sum<FT_N>(fbs[1]);
-  double ga = 0.0;
-#pragma unroll
-  for (int q = 0; q < FT_N; ++q) ga += dfa_in[q] * fbs[0][q];
-#pragma unroll
-  for (int q = 0; q < FT_N; ++q) {
-    fb_out[q] = fbs[0][q];
-    fbJ_io[q] += fbs[1][q];
-  }
-  return ga;
-}
-
 // One tangent direction per lane: lane & 7 == 0 carries d/da (component 0 of
 // TL, seeded by seed_tl), lane & 7 == c (1 <= c <= ndir) the input tangent
 // c - 1 (component 1, loaded through lane_ctx); TL arithmetic then costs
@@ -654,11 +670,14 @@ __device__ __forceinline__ double lane_dot(const TL (&F)[FT_N], const double (&f
 
 // feature values at a (plain doubles), wave-uniform: stored once per wave in
 // LDS (every lane writes the same values)
-DEB_OUTLINE void feature_values(Ctx &cx, double a, lds_double *fv) {
+template <int NS>
+DEB_OUTLINE void feature_values(Mode<NS> &m, Ctx &cx, double a, lds_double *fv) {
+  BgCache g;
+  const BgRow<double> b = mode_background<NS>(m, g, a);
   double f[FT_N];
-  features_t<double>(cx, a, f);
+  features_row(cx, g, b, f);
 #pragma unroll
-  for (int m = 0; m < FT_N; ++m) fv[m] = f[m];
+  for (int q = 0; q < FT_N; ++q) fv[q] = f[q];
 }
 
 // the lane's direction of sum_m F_m(a) fbs_m (fbs wave-uniform): d/da on
@@ -694,7 +713,7 @@ DEB_OUTLINE double lane_contract_stages(const Ctx &cx, const lds_double *cst) {
 // sums and the per-lane feature partials P (fb.v) with their a-derivatives Q
 // (fb.d), at the features of a.
 template <int NS>
-DEB_OUTLINE void acol_pass(Ctx &cx, const uint32_t (&rd)[NS], dual a, double invtau, const double (&w_in)[NS],
+DEB_OUTLINE void acol_pass(Mode<NS> &m, Ctx &cx, dual a, double invtau, const double (&w_in)[NS],
                            const double (&Y_in)[NS], dual (&out_io)[NS], dual (&fb_out)[FT_N]) {
   using T = dual;
   const int lane = lane_id();
@@ -704,15 +723,17 @@ DEB_OUTLINE void acol_pass(Ctx &cx, const uint32_t (&rd)[NS], dual a, double inv
     w[s] = w_in[s];
     Y[s] = Y_in[s];
   }
-  const Bg<T> b = background<T>(cx, a);
+  const RowK<NS> K = m.rk;
+  BgCache g;
+  const BgRow<T> b = mode_background<NS>(m, g, a);
   T F[1][FT_N];
-  features_of<T>(cx, a, b, F[0]);
+  features_row(cx, g, b, F[0]);
   T out[NS], part[7], cc[4][NS];
 #pragma unroll
   for (int i = 0; i < 7; ++i) part[i] = tconst<T>(0.0);
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    const Coef<T> r = row_coef_slot<T>(rd[s], b, cx, invtau, s == 0);
+    const Coef<T> r = row_lin<NS, T>(K, s, b, g, invtau);
     T sw = r.sub * w[s];
     T pw = r.sup * w[s];
     out[s] = r.diag * w[s] + t_from_next(sw) + t_from_prev(pw);
@@ -749,7 +770,7 @@ DEB_OUTLINE void acol_pass(Ctx &cx, const uint32_t (&rd)[NS], dual a, double inv
   T fb[1][FT_N];
 #pragma unroll
   for (int q = 0; q < FT_N; ++q) fb[0][q] = tconst<T>(0.0);
-  feature_partials_body<NS, 1, T>(cx, rd, F, Yd, wd, rs, fb);
+  feature_partials_body<NS, 1, T>(cx, m.rd, F, Yd, wd, rs, fb);
 #pragma unroll
   for (int q = 0; q < FT_N; ++q) fb_out[q] = fb[0][q];
 }
@@ -807,7 +828,7 @@ __device__ __forceinline__ RowSums jac_sums(const Mode<NS> &m, const double (&Y)
 // the stage's stored to fb_out and contracted with dfa into the a-direction of
 // ub (fbJ and fb_out: one copy per wave in LDS).
 template <int NS>
-DEB_OUTLINE void stage_rows(Ctx &cx, const Mode<NS> &m, double ai, double iti, const double (&rb_in)[NS],
+DEB_OUTLINE void stage_rows(Ctx &cx, Mode<NS> &m, double ai, double iti, const double (&rb_in)[NS],
                             const double (&u_in)[NS], const double (&ki_in)[NS], const lds_double *fvJ_in,
                             double (&ub_out)[NS], lds_double *fbJ_io, lds_double *fb_out) {
   const int lane = lane_id();
@@ -825,8 +846,22 @@ DEB_OUTLINE void stage_rows(Ctx &cx, const Mode<NS> &m, double ai, double iti, c
     fbs[0][q] = 0.0;
     fbs[1][q] = 0.0;
   }
+  // one background evaluation along a: its values for the rows, both for the features
   RowSums rsq[2];
-  rsq[0] = coef_pass_body<NS, true, true>(cx, m.rd, ai, iti, rb, u, ub, fvs[0], dfa);
+  {
+    const RowK<NS> K = m.rk;
+    BgCache g;
+    const BgRow<dual> bd = mode_background<NS>(m, g, mkd(ai, 1.0));
+    dual F[FT_N];
+    features_row(cx, g, bd, F);
+#pragma unroll
+    for (int q = 0; q < FT_N; ++q) {
+      fvs[0][q] = F[q].v;
+      dfa[q] = F[q].d;
+    }
+    const BgRow<double> b{bd.a.v, bd.aH.v, bd.iaH.v, bd.ia.v, bd.ia2.v, bd.opac.v, bd.cs2.v, bd.po.v, bd.rhoQ.v};
+    rsq[0] = coef_pass_body<NS>(K, g, b, iti, rb, u, ub);
+  }
   double Yq[2][NS], wq[2][NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
@@ -837,18 +872,17 @@ DEB_OUTLINE void stage_rows(Ctx &cx, const Mode<NS> &m, double ai, double iti, c
   }
   rsq[1] = jac_sums<NS>(m, ki, wq[1]);
   feature_partials_body<NS, 2>(cx, m.rd, fvs, Yq, wq, rsq, fbs);
-  wave_sum<FT_N>(fbs[0]);
-  wave_sum<FT_N>(fbs[1]);
   double ga = 0.0;
 #pragma unroll
   for (int q = 0; q < FT_N; ++q) ga += dfa[q] * fbs[0][q];
+  ga = wave_sum1(ga);
   if (lane == L_A) ub[0] += ga;
 #pragma unroll
   for (int s = 0; s < NS; ++s) ub_out[s] = ub[s];
-#pragma unroll
-  for (int q = 0; q < FT_N; ++q) {
-    fb_out[q] = fbs[0][q];
-    fbJ_io[q] += fbs[1][q];
+  const double t0 = wave_sum_spread(fbs[0]), t1 = wave_sum_spread(fbs[1]);
+  if (lane < FT_N) {
+    fb_out[lane] = t0;
+    fbJ_io[lane] += t1;
   }
 }
 
@@ -936,7 +970,7 @@ __device__ __forceinline__ void rodas5_step_vjp(Mode<NS> &m, Ctx &cx, double t0,
   // wave-uniform: one copy per wave in LDS (written by every lane alike)
   __shared__ double fvJ_[FT_N], fbJ_[FT_N];
   lds_double *const fvJ = (lds_double *)fvJ_, *const fbJl = (lds_double *)fbJ_;
-  feature_values(cx, a0, fvJ);
+  feature_values<NS>(m, cx, a0, fvJ);
 #pragma unroll
   for (int q = 0; q < FT_N; ++q) fbJl[q] = 0.0;
 #pragma nounroll
@@ -953,14 +987,14 @@ __device__ __forceinline__ void rodas5_step_vjp(Mode<NS> &m, Ctx &cx, double t0,
       ck[s] = 0.0;
     }
     // this stage's vector and the earlier ones in one batch of loads (the
-    // tableau's rows are zero from column i on, so the sums over all seven add
-    // exact zeros)
+    // tableau's rows are zero from column i on, so the sums add exact zeros
+    // there; stages 1 to 4 leave the last four columns out)
     {
       double kj[7][NS];
 #pragma unroll
       for (int j = 0; j < 7; ++j)
 #pragma unroll
-        for (int s = 0; s < NS; ++s) kj[j][s] = Kp(j, s);
+        for (int s = 0; s < NS; ++s) kj[j][s] = (j < 3 || i > 3) ? Kp(j, s) : 0.0;
 #pragma unroll
       for (int s = 0; s < NS; ++s) ki[s] = Kp(i, s);
 #pragma unroll
@@ -1001,27 +1035,7 @@ __device__ __forceinline__ void rodas5_step_vjp(Mode<NS> &m, Ctx &cx, double t0,
     double ub[NS];
     {
       const double ai = readlane(u[0], L_A);
-      if constexpr (NS <= 4) {
-        stage_rows<NS>(cx, m, ai, iti, rb, u, ki, fvJ, ub, fbJl, cst + 8 + i * FT_N);
-      } else {
-        // five slots: the same work as separate calls (as one call the
-        // reverse launch of the lmax-50 workload measured 14 % slower)
-        double fvs[FT_N], dfl[FT_N], Yq[2][NS], wq[2][NS];
-        RowSums rsq[2];
-        rsq[0] = coef_pass<NS, true, true>(cx, m.rd, ai, iti, rb, u, ub, fvs, dfl);
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-          Yq[0][s] = u[s];
-          wq[0][s] = rb[s];
-          Yq[1][s] = ki[s];
-          wq[1][s] = (s == 0 && lane == L_A) ? 0.0 : rb[s];
-        }
-        rsq[1] = jac_sums<NS>(m, ki, wq[1]);
-        // the a-direction now (it feeds the earlier stages); the input-tangent
-        // directions of all stages in one pass after the loop
-        const double ga = stage_partials<NS>(cx, m.rd, fvs, fvJ, dfl, Yq, wq, rsq, fbJl, cst + 8 + i * FT_N);
-        if (lane == L_A) ub[0] += ga;
-      }
+      stage_rows<NS>(cx, m, ai, iti, rb, u, ki, fvJ, ub, fbJl, cst + 8 + i * FT_N);
       cst[i] = ai;
       const double kia = readlane(ki[0], L_A);
 #pragma unroll
@@ -1035,6 +1049,7 @@ __device__ __forceinline__ void rodas5_step_vjp(Mode<NS> &m, Ctx &cx, double t0,
       for (int s = 0; s < NS; ++s) KBp(j, s) += aij * ub[s];
     }
   }
+  lds_sync();
   // the stages' input-tangent directions
   {
     const double g = lane_contract_stages(cx, cst);
@@ -1048,11 +1063,6 @@ __device__ __forceinline__ void rodas5_step_vjp(Mode<NS> &m, Ctx &cx, double t0,
       }
     }
   }
-  // the J(t0, y0) k_i terms' partials, contracted with the feature tangents
-  // at a0 together with the a-column's below (first order: added to Q)
-  double fbJ[FT_N];
-#pragma unroll
-  for (int q = 0; q < FT_N; ++q) fbJ[q] = fbJl[q];
   // a-column of J(t0, y0): rho^T df/da, differentiated along y0, a0 and theta
   {
     dual ad;
@@ -1061,24 +1071,27 @@ __device__ __forceinline__ void rodas5_step_vjp(Mode<NS> &m, Ctx &cx, double t0,
     // rho^T A'(a) (the derivative of the transposed apply), and for
     // S = rho^T f(a, y0) the per-lane feature partials in dual arithmetic
     dual gy[NS], fbd[FT_N];
-    acol_pass<NS>(cx, m.rd, ad, it0, rho, y0, gy, fbd);
+    acol_pass<NS>(m, cx, ad, it0, rho, y0, gy, fbd);
 #pragma unroll
     for (int s = 0; s < NS; ++s) y0b[s] += gy[s].d;
     // the feature partials P and their a-derivative Q, summed over the wave
     // and kept in the stage block (whose contraction has been read), then the
     // features' second derivatives
-    double PQ[2 * FT_N];
+    // (the J(t0, y0) k_i terms' partials join Q: contracted with the same
+    // feature tangents at a0, to first order)
+    double P[FT_N], Q[FT_N];
 #pragma unroll
     for (int q = 0; q < FT_N; ++q) {
-      PQ[q] = fbd[q].v;
-      PQ[FT_N + q] = fbd[q].d;
+      P[q] = fbd[q].v;
+      Q[q] = fbd[q].d;
     }
-    wave_sum<2 * FT_N>(PQ);
-#pragma unroll
-    for (int q = 0; q < FT_N; ++q) {
-      cst[q] = PQ[q];
-      cst[FT_N + q] = PQ[FT_N + q] + fbJ[q];
+    const double p = wave_sum_spread(P), q = wave_sum_spread(Q);
+    lds_sync();
+    if (lane < FT_N) {
+      cst[lane] = p;
+      cst[FT_N + lane] = q + fbJl[lane];
     }
+    lds_sync();
     const double g = lane_contract2(cx, a0, cst);
     a0b += readlane(g, 0);
     double tl[MAXDIR];
@@ -1247,12 +1260,6 @@ inline int output_inputs(const deb_config_t &c, int32_t *idx) {
   idx[m++] = n - 1;
   for (int i = m; i < WAVE; ++i) idx[i] = -1;
   return m;
-}
-
-__device__ __forceinline__ void lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
 // reverse of the output conversion of one output time: yb = dL/dy (slot

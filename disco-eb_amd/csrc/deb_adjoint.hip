@@ -114,7 +114,10 @@ __global__ void __launch_bounds__(WAVE) deb_rhs_vjp_kernel(const Params<NS> P_, 
   const double a = readlane(y[0], L_A);
   double fv[1][FT_N], fb[1][FT_N], Yq[1][NS], wq[1][NS];
   RowSums rs[1];
-  rs[0] = coef_pass<NS, true>(cx, rd, a, it, w, y, yb, fv[0]);
+  Mode<NS> m;
+  row_consts<NS>(rd, cx, m.rk);
+  bg_init(cx, m.bg);
+  rs[0] = coef_pass<NS>(m, cx, a, it, w, y, yb, fv[0]);
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
     Yq[0][s] = y[s];

@@ -408,6 +408,17 @@ __device__ __forceinline__ double row_sum16(double x) {
   return x;
 }
 #endif
+// the value of the lane that differs in bit B of its number within the row of
+// 16 and (B = 2, 3) in the bits below it too
+template <int B>
+__device__ __forceinline__ double row_partner(double x) {
+#ifdef DEB_NO_DPP
+  return from_lane(x, __lane_id() ^ (B == 3 ? 15 : (B == 2 ? 7 : 1 << B)));
+#else
+  constexpr int CTRL = B == 0 ? 0xB1 : (B == 1 ? 0x4E : (B == 2 ? 0x141 : 0x140));
+  return dpp_f64<CTRL, true>(x);
+#endif
+}
 template <int N>
 __device__ __forceinline__ void wave_sum(double (&v)[N]) {
   const int lane = lane_id();

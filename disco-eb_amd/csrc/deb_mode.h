@@ -541,19 +541,6 @@ __device__ __forceinline__ Coef<T> row_coef_wave(uint32_t d, const Bg<T> &b, con
   return r;
 }
 
-// row_coef of slot s: the wave form in plain doubles; dual arithmetic (the
-// factorisation's a-column and the reverse step's a-column) keeps the switch.
-// With the wave form also in the factorisation's dual right-hand side, the
-// fully inlined forward kernel ended 41 % of the headline modes at max_steps on
-// the GPU, although the host emulation finds the dual wave form equal to the
-// switch in every field; the cause was not found.
-template <typename T>
-__device__ __forceinline__ Coef<T> row_coef_slot(uint32_t d, const Bg<T> &b, const Ctx &cx, double invtau,
-                                                 bool slot0) {
-  if constexpr (std::is_same<T, double>::value) return row_coef_wave<T>(d, b, cx, invtau, slot0);
-  else return row_coef<T>(d, b, cx, invtau);
-}
-
 // ---------------------------------------------------------------------------
 // The rows as constants times background features.  Along one mode every
 // coefficient of a row is a number that depends on the row, k and the
