@@ -113,6 +113,11 @@ __device__ __forceinline__ void bsolveT(const Mode<NS> &m, double (&x)[NS]) {
   for (int L = PCR_LEVELS - 1; L >= 0; --L) {
     if (L >= m.nlev) continue;
     const int s = 1 << L;
+    if (L == PCR_LAST) {
+#pragma unroll
+      for (int j = 0; j < NS; ++j) x[j] += from_lane(m.al(L, j) * x[j], lane ^ 32);
+      continue;
+    }
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
       const double v = m.al(L, j) * x[j];
@@ -151,14 +156,14 @@ DEB_OUTLINE void wsolveT(const Mode<NS> &m, double (&xio)[NS]) {
   const double r1b = m.u->gh * kb1;
   double kab = kba + m.u->gh * m.u->J1a * kb1;
   const double c1kb = m.u->gh * kb1;
-  double part[3] = {0.0, 0.0, 0.0};
+  double part[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
     part[0] += m.Z[0][s] * x[s];
     part[1] += m.Z[1][s] * x[s];
     part[2] += m.Z[2][s] * x[s];
   }
-  wave_sum<3>(part);
+  wave_sum4(part);
   double tt[3];
 #pragma unroll
   for (int r = 0; r < 3; ++r) tt[r] = m.u->c1Z[r] * c1kb + part[r];
@@ -264,26 +269,6 @@ __device__ __forceinline__ BgRow<T> mode_background(Mode<NS> &m, BgCache &g, T a
   return b;
 }
 
-// The 16 sums over the wave of v, one per lane: lane l returns that of
-// v[l & 15].  The butterfly of wave_sum with the values split between the
-// partners at each of the row's four exchanges: 111 instructions, where 16
-// whole sums take 288.
-__device__ __forceinline__ double wave_sum_spread(const double (&v)[16]) {
-  const int lane = lane_id();
-  const bool b3 = (lane & 8) != 0, b2 = (lane & 4) != 0, b1 = (lane & 2) != 0, b0 = (lane & 1) != 0;
-  double w[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) w[i] = (b3 ? v[i + 8] : v[i]) + row_partner<3>(b3 ? v[i] : v[i + 8]);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) w[i] = (b2 ? w[i + 4] : w[i]) + row_partner<2>(b2 ? w[i] : w[i + 4]);
-#pragma unroll
-  for (int i = 0; i < 2; ++i) w[i] = (b1 ? w[i + 2] : w[i]) + row_partner<1>(b1 ? w[i] : w[i + 2]);
-  double r = (b0 ? w[1] : w[0]) + row_partner<0>(b0 ? w[0] : w[1]);
-  r += from_lane(r, lane ^ 16);
-  r += from_lane(r, lane ^ 32);
-  return r;
-}
-
 // Values of the functionals of Y and of the "where they enter" sums of w that
 // the first-order contraction below needs, plus (optionally) the transposed
 // right-hand side A(a)^T w -- one plain-double pass over the rows.
@@ -300,7 +285,7 @@ __device__ __forceinline__ RowSums coef_pass_body(const RowK<NS> &K, const BgCac
                                                   double (&out)[NS]) {
   const int lane = lane_id();
   double o[NS];
-  double part[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  double part[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   double cc[4][NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
@@ -324,7 +309,7 @@ __device__ __forceinline__ RowSums coef_pass_body(const RowK<NS> &K, const BgCac
     cc[2][s] = r.cpi;
     cc[3][s] = r.c1;
   }
-  wave_sum<7>(part);
+  wave_sum8(part);
   RowSums rs{part[0], part[1], part[2], part[3], part[4], part[5], part[6]};
   const double wahp = readlane(w[0], L_AHP);
 #pragma unroll
@@ -805,7 +790,7 @@ __device__ __forceinline__ void lane_gather(double g, int ndir, double (&out)[MA
 // row sums of the step Jacobian J(t0, y0) kept by the factorisation
 template <int NS>
 __device__ __forceinline__ RowSums jac_sums(const Mode<NS> &m, const double (&Y)[NS], const double (&w)[NS]) {
-  double part[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  double part[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
     part[0] += m.Cf[0][s] * Y[s];
@@ -816,7 +801,7 @@ __device__ __forceinline__ RowSums jac_sums(const Mode<NS> &m, const double (&Y)
     part[5] += m.U[1][s] * w[s];
     part[6] += m.U[2][s] * w[s];
   }
-  wave_sum<7>(part);
+  wave_sum8(part);
   return RowSums{part[0], part[1], part[2], part[3], part[4], part[5], part[6]};
 }
 
@@ -1016,14 +1001,14 @@ __device__ __forceinline__ void rodas5_step_vjp(Mode<NS> &m, Ctx &cx, double t0,
     const double iti = 1.0 / ti;
     // dot products: h-derivative of W, C/h and d h dT terms; explicit time
     // dependence at the stage point and of J at (t0, y0)
-    double dots[3] = {0.0, 0.0, 0.0};
+    double dots[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       dots[0] += rb[s] * (ki[s] / (gamma * h * h) - ck[s] * ih * ih + kd[i] * dT[s]);
       dots[1] += rb[s] * tw[s] * iti * iti * u[s];
       dots[2] += rb[s] * tw[s] * it0 * it0 * ki[s];
     }
-    wave_sum<3>(dots);
+    wave_sum4(dots);
     hb += dots[0] + kc[i] * dots[1];
     t0b += dots[1] + dots[2];
     if (kd[i] != 0.0) {

@@ -24,6 +24,8 @@ namespace deb {
 constexpr int WAVE = 64;
 constexpr int MAXNS = 6;
 constexpr int PCR_LEVELS = 6;
+// the last level couples lane i to lane i ^ 32 only (one coefficient per row)
+constexpr int PCR_LAST = 5;
 
 // pointers into a wave's LDS (address space 3: ds_read/ds_write, also inside
 // outlined functions, which would otherwise address LDS with flat instructions)
@@ -33,10 +35,10 @@ constexpr int PCR_LEVELS = 6;
 typedef DEB_LDS double lds_double;
 
 // doubles of LDS one wave needs for its step factors: the cyclic-reduction
-// coefficients (alpha, beta) of every level and row
+// coefficients (alpha, beta; one at the last level) of every level and row
 template <int NS>
 constexpr int pcr_lds_doubles() {
-  return PCR_LEVELS * 2 * NS * WAVE;
+  return (PCR_LEVELS * 2 - 1) * NS * WAVE;
 }
 
 // the forward kernels keep the step's 7 stage vectors in LDS where the wave's
@@ -428,6 +430,59 @@ __device__ __forceinline__ void wave_sum(double (&v)[N]) {
   for (int i = 0; i < N; ++i) v[i] += from_lane(v[i], lane ^ 16);
 #pragma unroll
   for (int i = 0; i < N; ++i) v[i] += from_lane(v[i], lane ^ 32);
+}
+// The 16 sums over the wave of v, one per lane: lane l returns that of
+// v[l & 15].  The butterfly of wave_sum with the values split between the
+// partners at each of the row's four exchanges: 111 instructions, where 16
+// whole sums take 288.
+__device__ __forceinline__ double wave_sum_spread(const double (&v)[16]) {
+  const int lane = lane_id();
+  const bool b3 = (lane & 8) != 0, b2 = (lane & 4) != 0, b1 = (lane & 2) != 0, b0 = (lane & 1) != 0;
+  double w[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) w[i] = (b3 ? v[i + 8] : v[i]) + row_partner<3>(b3 ? v[i] : v[i + 8]);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = (b2 ? w[i + 4] : w[i]) + row_partner<2>(b2 ? w[i] : w[i + 4]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) w[i] = (b1 ? w[i + 2] : w[i]) + row_partner<1>(b1 ? w[i] : w[i + 2]);
+  double r = (b0 ? w[1] : w[0]) + row_partner<0>(b0 ? w[0] : w[1]);
+  r += from_lane(r, lane ^ 16);
+  r += from_lane(r, lane ^ 32);
+  return r;
+}
+// Four wave-wide sums, wave-uniform.  The values are split between the partners
+// of the row's first two exchanges, so that the last four exchanges carry one
+// value: 41 instructions and 4 LDS moves, where wave_sum<4> takes 72 and 16.
+__device__ __forceinline__ void wave_sum4(double (&v)[4]) {
+  const int lane = lane_id();
+  const bool b3 = (lane & 8) != 0, b2 = (lane & 4) != 0;
+  const double w0 = (b3 ? v[2] : v[0]) + row_partner<3>(b3 ? v[0] : v[2]);
+  const double w1 = (b3 ? v[3] : v[1]) + row_partner<3>(b3 ? v[1] : v[3]);
+  double r = (b2 ? w1 : w0) + row_partner<2>(b2 ? w0 : w1);
+  r += row_partner<1>(r);
+  r += row_partner<0>(r);
+  r += from_lane(r, lane ^ 16);
+  r += from_lane(r, lane ^ 32);
+  v[0] = readlane(r, 0);
+  v[1] = readlane(r, 4);
+  v[2] = readlane(r, 8);
+  v[3] = readlane(r, 12);
+}
+// Eight wave-wide sums, wave-uniform (72 instructions, whole sums 144).
+__device__ __forceinline__ void wave_sum8(double (&v)[8]) {
+  const int lane = lane_id();
+  const bool b3 = (lane & 8) != 0, b2 = (lane & 4) != 0, b1 = (lane & 2) != 0;
+  double w[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = (b3 ? v[i + 4] : v[i]) + row_partner<3>(b3 ? v[i] : v[i + 4]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) w[i] = (b2 ? w[i + 2] : w[i]) + row_partner<2>(b2 ? w[i] : w[i + 2]);
+  double r = (b1 ? w[1] : w[0]) + row_partner<1>(b1 ? w[0] : w[1]);
+  r += row_partner<0>(r);
+  r += from_lane(r, lane ^ 16);
+  r += from_lane(r, lane ^ 32);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = readlane(r, 8 * (i >> 2) + 4 * ((i >> 1) & 1) + 2 * (i & 1));
 }
 // one wave-wide sum, returned as a wave-uniform (scalar) value
 __device__ __forceinline__ double wave_sum1(double x) {

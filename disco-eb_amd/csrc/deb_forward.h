@@ -261,6 +261,18 @@ struct TapeWriter {
 // shrinks it by factormin
 __device__ __forceinline__ double norm_or_inf(double nrm) { return nrm <= 1.7976931348623157e308 ? nrm : INFINITY; }
 
+// 0.9 inv^c1 prev^c2 prevprev^c3, the controller's factor: lanes 0..2 of each four
+// take one power each, so that a step costs one pow instead of three (a zero
+// exponent's factor is exactly 1)
+__device__ __forceinline__ double pid_factor(double inv, double prev, double prevprev, double c1, double c2,
+                                             double c3) {
+  const int j = lane_id() & 3;
+  const double b = j == 0 ? inv : (j == 1 ? prev : prevprev);
+  const double c = j == 0 ? c1 : (j == 1 ? c2 : c3);
+  const double f = c == 0.0 ? 1.0 : pow(b, c);
+  return 0.9 * readlane(f, 0) * readlane(f, 1) * readlane(f, 2);
+}
+
 // true on every lane if any lane holds a non-finite state entry
 template <int NS>
 __device__ __forceinline__ bool any_nonfinite(const double (&y)[NS]) {
@@ -356,11 +368,8 @@ __device__ __forceinline__ void integrate_mode(const Params<NS> &P, int ci, int 
     const double nrm = norm_or_inf(sqrt(wave_sum1(x * x) / 6.0));
     const bool keep = nrm < 1.0;
     double inv = 1.0 / nrm;
-    double f1 = coeff1 == 0.0 ? 1.0 : pow(inv, coeff1);
-    double f2 = coeff2 == 0.0 ? 1.0 : pow(prev_inv, coeff2);
-    double f3 = coeff3 == 0.0 ? 1.0 : pow(prev_prev_inv, coeff3);
     double fmn = keep ? 1.0 : cf.factormin;
-    double factor = fmin(fmax(0.9 * f1 * f2 * f3, fmn), cf.factormax);
+    double factor = fmin(fmax(pid_factor(inv, prev_inv, prev_prev_inv, coeff1, coeff2, coeff3), fmn), cf.factormax);
     double dtn = dt * factor;
     if (inv == 0.0 || isinf(inv)) inv = 1.0;
     if (keep) {
@@ -492,11 +501,8 @@ __device__ __forceinline__ void integrate_batch(const Params<NS> &P, int ci, int
     const double nrm = norm_or_inf(sqrt(e2 / (6.0 * B)));
     const bool keep = nrm < 1.0;
     double inv = 1.0 / nrm;
-    double f1 = coeff1 == 0.0 ? 1.0 : pow(inv, coeff1);
-    double f2 = coeff2 == 0.0 ? 1.0 : pow(prev_inv, coeff2);
-    double f3 = coeff3 == 0.0 ? 1.0 : pow(prev_prev_inv, coeff3);
     double fmn = keep ? 1.0 : cf.factormin;
-    double factor = fmin(fmax(0.9 * f1 * f2 * f3, fmn), cf.factormax);
+    double factor = fmin(fmax(pid_factor(inv, prev_inv, prev_prev_inv, coeff1, coeff2, coeff3), fmn), cf.factormax);
     double dtn = dt * factor;
     if (inv == 0.0 || isinf(inv)) inv = 1.0;
     if (keep) {

@@ -80,7 +80,8 @@ __device__ __forceinline__ void eval_rhs(BgCache &bg, const RowK<NS> &K, double 
       part[7] += dval(cf[s].c1) * y[s];
     }
   }
-  wave_sum<NV>(part);
+  if constexpr (NV == 4) wave_sum4(part);
+  else wave_sum<NV>(part);
   T hp, etap, Pi, f1;
   if constexpr (NV == 8) {
     hp = T{part[0], part[4]};
@@ -134,6 +135,11 @@ __device__ __forceinline__ void bsolve(const Mode<NS> &m, double (&x)[NS]) {
   for (int L = 0; L < PCR_LEVELS; ++L) {
     if (L >= m.nlev) break;
     const int s = 1 << L;
+    if (L == PCR_LAST) {
+#pragma unroll
+      for (int j = 0; j < NS; ++j) x[j] += m.al(L, j) * from_lane(x[j], lane ^ 32);
+      break;
+    }
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
       double dm, dp;
@@ -200,11 +206,24 @@ __device__ __forceinline__ void factor(Mode<NS> &m, double tau0, const double (&
   // is eliminated at level 0 by cross-multiplication (its theta_Q pivot can
   // vanish), every other row by the usual reduction, which multiplies by the
   // neighbours' pivot reciprocals (each lane takes the reciprocal of its own
-  // pivot once per level; rows not coupled to a neighbour never use it)
+  // pivot once per level).  A row that is not coupled to a neighbour has a zero
+  // coefficient, so its products vanish; only the dark-energy pivots of slot 0
+  // can be infinite there, and those are guarded at level 0.
 #pragma unroll
   for (int L = 0; L < PCR_LEVELS; ++L) {
     if (L >= m.nlev) break;
     const int s = 1 << L;
+    if (L == PCR_LAST) {
+      // lanes below 32 have only the neighbour above, the others only the one below
+#pragma unroll
+      for (int j = 0; j < NS; ++j) {
+        const double E = lane < 32 ? Cc[j] : A[j];
+        const double al = -E * from_lane(rcp_nr(Bd[j]), lane ^ 32);
+        m.al(L, j) = al;
+        Bd[j] += al * from_lane(E, lane ^ 32);
+      }
+      break;
+    }
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
       const double ib = rcp_nr(Bd[j]);
@@ -218,8 +237,11 @@ __device__ __forceinline__ void factor(Mode<NS> &m, double tau0, const double (&
         am = from_lane(A[j], lm); ibm = from_lane(ib, lm); cm = from_lane(Cc[j], lm);
         ap = from_lane(A[j], lp); ibp = from_lane(ib, lp); cp = from_lane(Cc[j], lp);
       }
-      double alpha = (A[j] == 0.0) ? 0.0 : -A[j] * ibm;
-      double beta = (Cc[j] == 0.0) ? 0.0 : -Cc[j] * ibp;
+      double alpha = -A[j] * ibm, beta = -Cc[j] * ibp;
+      if (L == 0 && j == 0) {
+        alpha = A[j] == 0.0 ? 0.0 : alpha;
+        beta = Cc[j] == 0.0 ? 0.0 : beta;
+      }
       double sg = 1.0;
       if (L == 0 && j == 0) {
         // scale the row by the partner's pivot instead of dividing by it
@@ -254,9 +276,9 @@ __device__ __forceinline__ void factor(Mode<NS> &m, double tau0, const double (&
 #pragma unroll
     for (int s = 0; s < NS; ++s) m.Z[r][s] = x[s];
   }
-  double part[12];
+  double part[16];
 #pragma unroll
-  for (int i = 0; i < 12; ++i) part[i] = 0.0;
+  for (int i = 0; i < 16; ++i) part[i] = 0.0;
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
 #pragma unroll
@@ -266,7 +288,11 @@ __device__ __forceinline__ void factor(Mode<NS> &m, double tau0, const double (&
       part[9 + r] += m.c1[s] * m.Z[r][s];
     }
   }
-  wave_sum<12>(part);
+  {
+    const double t = wave_sum_spread(part);
+#pragma unroll
+    for (int i = 0; i < 12; ++i) part[i] = readlane(t, i);
+  }
   double S[3][3];
 #pragma unroll
   for (int r = 0; r < 3; ++r)
@@ -309,7 +335,7 @@ __device__ __forceinline__ void wsolve(const Mode<NS> &m, double (&r)[NS]) {
     g[2] += m.Cf[2][s] * r[s];
     g[3] += m.c1[s] * r[s];
   }
-  wave_sum<4>(g);
+  wave_sum4(g);
   double t[3];
 #pragma unroll
   for (int i = 0; i < 3; ++i) t[i] = m.u->Sinv[i][0] * g[0] + m.u->Sinv[i][1] * g[1] + m.u->Sinv[i][2] * g[2];
@@ -420,7 +446,7 @@ __device__ __forceinline__ void rodas5_step_s(Mode<NS> &m, double t0, double dt,
       double du[NS];
 #pragma unroll
       for (int s = 0; s < NS; ++s) du[s] = i >= 6 ? u[s] + k[s] : y0[s];
-      const double la = i >= 6 ? 0.0 : 1.0;
+      const int ia = i >= 6 ? 0 : i;  // row 0 of the tableau is zero
       auto add = [&](auto first, auto count) {
         constexpr int J0 = decltype(first)::value, NJ = decltype(count)::value;
         double kj[NJ][NS];
@@ -430,7 +456,7 @@ __device__ __forceinline__ void rodas5_step_s(Mode<NS> &m, double t0, double dt,
           for (int s = 0; s < NS; ++s) kj[j][s] = K(J0 + j, s);
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-          const double aij = la * kA[i][J0 + j], cij = kC[i][J0 + j];
+          const double aij = kA[ia][J0 + j], cij = kC[i][J0 + j];
 #pragma unroll
           for (int s = 0; s < NS; ++s) {
             if (J0 + j < 5) du[s] += aij * kj[j][s];
