@@ -338,287 +338,112 @@ DEB_OUTLINE RowSums coef_pass(Mode<NS> &m, Ctx &cx, double a, double invtau, con
   return rs;
 }
 
-// Partials of the rows' sum_fields mul[q][f] coef_f with respect to the
-// features (accumulated into fb[q]) and to their bin velocity (vb[q]), for K
-// contractions at once; fv[q]: the feature values of contraction q.  The
-// partials of row_visit's formulas, organised for the wave rather than as one
-// divergent switch over row types:
-//   chain_feature_adj    the rows of the hierarchies (any slot, any lane):
-//                        per-lane arithmetic with selects, no branches;
-//   special_feature_adj  the rows that sit on fixed lanes of slot 0 (eta,
-//                        delta_c, theta_c, delta_b, theta_b, delta_gamma,
-//                        theta_gamma, delta_Q, theta_Q): their multipliers are
-//                        read from those lanes and their partials formed as
-//                        wave-uniform values, to be added once (on lane 0).
-template <int K, class T = double>
-__device__ __forceinline__ void chain_feature_adj(uint32_t d, const Ctx &cx, const T (&fv)[K][FT_N],
-                                                  const T (&vq)[K], const T (&mul)[K][11], T (&fb)[K][FT_N],
-                                                  T (&vb)[K]) {
-  const double k = cx.k, k2 = k * k;
-  const double hk2 = 0.5 / k2;
-  const uint32_t t = rd_type(d);
-  const double l = (double)rd_l(d);
-  // opacity through the diagonal (-opac) and the polarization source (c opac)
-  const bool od = t == R_F2 || t == R_FL || t == R_FLMAX || t == R_G0 || t == R_GL || t == R_G2 || t == R_GLMAX;
-  const double cu = (t == R_F2 || t == R_G2) ? 0.1 : (t == R_G0 ? 0.5 : 0.0);
-  // massive-nu rows: sub, sup proportional to k v_q
-  const bool qr = t >= R_Q0 && t <= R_QLMAX;
-  const double il = rcp_nr(2.0 * l + 1.0);
-  const double cs = t == R_Q1 ? 1.0 / 3.0 : (t == R_Q2 ? 0.4 : (t == R_QL ? l * il : (t == R_QLMAX ? 1.0 : 0.0)));
-  const double cp = t == R_Q0 ? 1.0 : (t == R_Q1 ? 2.0 / 3.0 : (t == R_Q2 ? 0.6 : (t == R_QL ? (l + 1.0) * il : 0.0)));
-  const bool q0 = t == R_Q0, q1 = t == R_Q1, dr = t == R_DR, tr = t == R_TR;
-  const double wq = (q0 || q1) ? cx.w[rd_q(d)] : 0.0;
-  const T zero = tconst<T>(0.0);
-#pragma unroll
-  for (int q = 0; q < K; ++q) {
-    const T *m = mul[q];
-    const T *F = fv[q];
-    if (od) fb[q][FT_OPAC] += -m[C_DIAG] + (cu != 0.0 ? cu * m[C_UPI] : zero);
-    if (qr) vb[q] += k * (m[C_SUB] * cs - m[C_SUP] * cp);
-    if (q0) {
-      // ch = RN wq / v * iaH; c1 = -a (RN wq / v + RN wq v)
-      const T RN = F[FT_RN];
-      const T iv = rcp_t<T>(vq[q]);
-      fb[q][FT_RN] += m[C_CH] * wq * iv * F[FT_IAH] - m[C_C1] * F[FT_A] * wq * (iv + vq[q]);
-      fb[q][FT_IAH] += m[C_CH] * RN * wq * iv;
-      vb[q] += -m[C_CH] * RN * wq * F[FT_IAH] * iv * iv - m[C_C1] * F[FT_A] * RN * wq * (1.0 - iv * iv);
-      fb[q][FT_A] += -m[C_C1] * RN * wq * (iv + vq[q]);
-    }
-    if (q1) fb[q][FT_RN] += m[C_CETA] * k * wq * hk2;
-    if (dr) {
-      fb[q][FT_RR] += m[C_CH] * F[FT_IAH] - 2.0 * m[C_C1] * F[FT_A];
-      fb[q][FT_IAH] += m[C_CH] * F[FT_RR];
-      fb[q][FT_A] += -2.0 * m[C_C1] * F[FT_RR];
-    }
-    if (tr) fb[q][FT_RR] += m[C_CETA] * (4.0 / 3.0) * hk2;
-  }
-}
-
-// the fixed-lane rows of slot 0 (multipliers ms0 of slot 0): wave-uniform
-// partials added into sp
-template <int K, class T = double>
-__device__ __forceinline__ void special_feature_adj(const Ctx &cx, const T (&fv)[K][FT_N], const T (&ms0)[K][11],
-                                                    T (&sp)[K][FT_N]) {
-  const double k = cx.k, k2 = k * k;
-  const double ik2 = 1.0 / k2, hk2 = 0.5 * ik2;
-#pragma unroll
-  for (int q = 0; q < K; ++q) {
-    const T *F = fv[q];
-    auto M = [&](int lane, int f) { return t_readlane(ms0[q][f], lane); };
-    T *o = sp[q];
-    // eta: ch = 2 k^2 iaH
-    o[FT_IAH] += M(L_ETA, C_CH) * 2.0 * k2;
-    // delta_c, delta_b: ch = R iaH, c1 = -a R (R = rho_c / a, rho_b / a)
-    {
-      const T ch = M(L_DC, C_CH), c1 = M(L_DC, C_C1);
-      o[FT_RC] += ch * F[FT_IAH] - c1 * F[FT_A];
-      o[FT_IAH] += ch * F[FT_RC];
-      o[FT_A] += -c1 * F[FT_RC];
-    }
-    {
-      const T ch = M(L_DB, C_CH), c1 = M(L_DB, C_C1);
-      o[FT_RB] += ch * F[FT_IAH] - c1 * F[FT_A];
-      o[FT_IAH] += ch * F[FT_RB];
-      o[FT_A] += -c1 * F[FT_RB];
-    }
-    // theta_c: diag = -aH, ceta = R_c hk2
-    o[FT_AH] += -M(L_TC, C_DIAG);
-    o[FT_RC] += M(L_TC, C_CETA) * hk2;
-    // theta_b: sub = k^2 cs2, diag = -aH - pb43 opac, sup = pb43 opac, ceta = R_b hk2
-    {
-      const T sub = M(L_TB, C_SUB), dg = M(L_TB, C_DIAG), sup = M(L_TB, C_SUP);
-      o[FT_CS2] += sub * k2;
-      o[FT_AH] += -dg;
-      o[FT_PB43] += (sup - dg) * F[FT_OPAC];
-      o[FT_OPAC] += (sup - dg) * F[FT_PB43];
-      o[FT_RB] += M(L_TB, C_CETA) * hk2;
-    }
-    // delta_gamma: ch = R_g iaH, c1 = -2 a R_g
-    {
-      const T ch = M(L_DG, C_CH), c1 = M(L_DG, C_C1);
-      o[FT_RG] += ch * F[FT_IAH] - 2.0 * c1 * F[FT_A];
-      o[FT_IAH] += ch * F[FT_RG];
-      o[FT_A] += -2.0 * c1 * F[FT_RG];
-    }
-    // theta_gamma: sub = opac, diag = -opac, ceta = (4/3) R_g hk2
-    o[FT_OPAC] += M(L_TG, C_SUB) - M(L_TG, C_DIAG);
-    o[FT_RG] += M(L_TG, C_CETA) * (4.0 / 3.0) * hk2;
-    if (!cx.lambda) {
-      const T w = F[FT_W], ca2 = F[FT_CA2], cs2Q = F[FT_CS2Q], RQ = F[FT_RQ];
-      const T opw = 1.0 + w;
-      {  // delta_Q
-        const T dg = M(L_DQ, C_DIAG), sup = M(L_DQ, C_SUP), uh = M(L_DQ, C_UH), ch = M(L_DQ, C_CH),
-                c1 = M(L_DQ, C_C1);
-        const T g = F[FT_AH] * F[FT_AH] * ik2;
-        // diag = -3 (cs2Q - w) aH
-        o[FT_CS2Q] += -3.0 * F[FT_AH] * dg;
-        o[FT_W] += 3.0 * F[FT_AH] * dg;
-        o[FT_AH] += -3.0 * (cs2Q - w) * dg;
-        // sup = -opw - 9 opw (cs2Q - ca2) aH^2 / k2
-        o[FT_W] += sup * (-1.0 - 9.0 * (cs2Q - ca2) * g);
-        o[FT_CS2Q] += -9.0 * opw * g * sup;
-        o[FT_CA2] += 9.0 * opw * g * sup;
-        o[FT_AH] += -18.0 * opw * (cs2Q - ca2) * F[FT_AH] * ik2 * sup;
-        // uh = -0.5 opw
-        o[FT_W] += -0.5 * uh;
-        // ch = RQ iaH
-        o[FT_RQ] += ch * F[FT_IAH];
-        o[FT_IAH] += ch * RQ;
-        // c1 = -a (RQ + 3 cs2Q RQ)
-        o[FT_A] += -c1 * RQ * (1.0 + 3.0 * cs2Q);
-        o[FT_RQ] += -c1 * F[FT_A] * (1.0 + 3.0 * cs2Q);
-        o[FT_CS2Q] += -c1 * 3.0 * F[FT_A] * RQ;
-      }
-      {  // theta_Q
-        const T sub = M(L_TQ, C_SUB), dg = M(L_TQ, C_DIAG), ce = M(L_TQ, C_CETA), c1 = M(L_TQ, C_C1);
-        // sub = cs2Q / opw k2
-        const T iopw = rcp_t<T>(opw);
-        o[FT_CS2Q] += sub * k2 * iopw;
-        o[FT_W] += -sub * cs2Q * k2 * (iopw * iopw);
-        // diag = -(1 - 3 cs2Q) aH
-        o[FT_CS2Q] += 3.0 * F[FT_AH] * dg;
-        o[FT_AH] += -(1.0 - 3.0 * cs2Q) * dg;
-        // ceta = opw RQ 0.5 / k2
-        o[FT_W] += ce * RQ * hk2;
-        o[FT_RQ] += ce * opw * hk2;
-        // c1 = -a 9 (cs2Q - ca2) aH opw RQ / k2
-        const double c9 = 9.0 * ik2;
-        o[FT_A] += -c1 * c9 * (cs2Q - ca2) * F[FT_AH] * opw * RQ;
-        o[FT_CS2Q] += -c1 * F[FT_A] * c9 * F[FT_AH] * opw * RQ;
-        o[FT_CA2] += c1 * F[FT_A] * c9 * F[FT_AH] * opw * RQ;
-        o[FT_AH] += -c1 * F[FT_A] * c9 * (cs2Q - ca2) * opw * RQ;
-        o[FT_W] += -c1 * F[FT_A] * c9 * (cs2Q - ca2) * F[FT_AH] * RQ;
-        o[FT_RQ] += -c1 * F[FT_A] * c9 * (cs2Q - ca2) * F[FT_AH] * opw;
-      }
-    }
-  }
-}
-
-// First-order contraction of sum_rows w_row f_row(a, Y) along (a, theta):
-//   slot_muls          the multiplier of every coefficient field of a row;
-//   feature_partials   per lane, the partials of its rows' sum_fields
-//                      mul * coef with respect to the features, accumulated
-//                      into fb (plain doubles, no cross-lane sums; linear in
-//                      mul, so contractions at the same features may share fb);
-//   lane_dot           after fb is summed over the wave, sum_m dF_m fb_m for
-//                      the lane's own tangent direction (lane_ctx).
-// The functionals (h', eta', Pi, f_1) enter through their double values in rs,
-// which is exact at first order: d(u H) = du H + u dH with dH = sum_rows dc_h Y,
-// so sum_rows w u dH = s_h sum_rows dc_h Y (multiplier Y s_h of the c_h field).
-
-// multipliers of the coefficient fields of slot s's rows in
-// sum_rows w f_row(Y) (the contraction's per-row weights): ys, ws the slot's
-// values, ym, yp its neighbours' (lanes i-1, i+1), ydg, ytg, wahp the
-// wave-uniform Y[L_DG], Y[L_TG], w[L_AHP] of slot 0; rs the functionals' values
-template <class T>
-__device__ __forceinline__ void slot_muls(int s, double ys, double ws, double ym, double yp, double ydg, double ytg,
-                                          double wahp, const RowSumsT<T> &rs, T (&ms)[11]) {
-  const int lane = lane_id();
-  const double lp = (s == 0) ? (lane == L_DG ? ytg : (lane == L_TG ? ydg : 0.0)) : 0.0;
-  ms[C_SUB] = tconst<T>(ws * ym);
-  ms[C_DIAG] = tconst<T>(ws * ys);
-  ms[C_SUP] = tconst<T>(ws * yp);
-  ms[C_UH] = ws * rs.H;
-  ms[C_UETA] = ws * rs.E;
-  ms[C_UPI] = ws * rs.Pi;
-  ms[C_CH] = ys * rs.sh;
-  ms[C_CETA] = ys * rs.se;
-  ms[C_CPI] = ys * rs.sp;
-  ms[C_C1] = tconst<T>(ys * wahp);
-  // the leaf field is unused by the a-row: there it carries the row weight w_a
-  ms[C_LEAF] = tconst<T>((s == 0 && lane == L_A) ? ws : ws * lp);
-}
-
-// fb[q] += partials, with respect to the features fv[q], of
-// sum_rows sum_fields mul_q coef_field, mul_q the row multipliers of
-// sum_rows w[q] f_row(Y[q]) (slot_muls, formed slot by slot here; rs[q] the
-// functionals' values): K contractions in one pass of the divergent row switch
+// First-order contraction of S = sum_rows w_row f_row(a, Y): its partials with
+// respect to the features, wave-uniform, for K contractions at once (fv[q] the
+// feature values of contraction q).  The functionals (h', eta', Pi, f_1) enter
+// through their values in rs, which is exact at first order: d(u H) = du H +
+// u dH with dH = sum_rows dc_h Y, so sum_rows w u dH = s_h sum_rows dc_h Y.
+//
+// Only four partials need the lanes: the opacity, the massive and massless
+// neutrino densities and the bin velocities (their -x dv/dx, x = a m_nu / q,
+// carries both the a and the m_nu partial).  c_h is proportional to 1/aH and
+// c_1 to a on every row, so those partials are s_h H and w_{ah'} f_1 over the
+// feature; the remaining rows sit on fixed lanes of slot 0 and are combined as
+// wave-uniform values read from there.  (Summed as 16 features per contraction
+// from per-row multipliers, a stage's two contractions took 2400 instructions;
+// this form takes about 700.)
 template <int NS, int K, class T = double>
-__device__ __forceinline__ void feature_partials_body(const Ctx &cx, const uint32_t (&rd)[NS],
-                                                      const T (&fv_in)[K][FT_N], const double (&Y_in)[K][NS],
-                                                      const double (&w_in)[K][NS], const RowSumsT<T> (&rs_in)[K],
-                                                      T (&fb)[K][FT_N]) {
-  const int lane = lane_id();
-  // Private copies: fb may alias the inputs as far as the compiler knows, so
-  // accumulating through the references would reload every operand after each
-  // store (memory traffic in the caller's frame); locals stay in registers.
-  T fv[K][FT_N], acc[K][FT_N];
-  double Y[K][NS], w[K][NS];
-  RowSumsT<T> rs[K];
-  double ydg[K], ytg[K], wahp[K];
+__device__ __forceinline__ void feature_totals(const Ctx &cx, const RowK<NS> &R, const uint32_t (&rd)[NS],
+                                               const T (&fv)[K][FT_N], const double (&Y)[K][NS],
+                                               const double (&w)[K][NS], const RowSumsT<T> (&rs)[K],
+                                               T (&fb)[K][FT_N]) {
+  constexpr int C = ncomp<T>::value;
+  static_assert(4 * K * C <= 8, "four lane sums per contraction");
+  const double k2 = cx.k * cx.k, ik2 = 1.0 / k2, hk2 = 0.5 * ik2;
+  T acc[K][4];  // opacity, velocity, massive and massless nu density
 #pragma unroll
   for (int q = 0; q < K; ++q) {
+    const T *F = fv[q];
+    const double wahp = readlane(w[q][0], L_AHP);
+    const T shi = rs[q].sh * F[FT_IAH], wa = wahp * F[FT_A];
 #pragma unroll
-    for (int m = 0; m < FT_N; ++m) {
-      fv[q][m] = fv_in[q][m];
-      acc[q][m] = tconst<T>(0.0);
-    }
+    for (int i = 0; i < 4; ++i) acc[q][i] = tconst<T>(0.0);
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      Y[q][s] = Y_in[q][s];
-      w[q][s] = w_in[q][s];
-    }
-    rs[q] = rs_in[q];
-    ydg[q] = readlane(Y[q][0], L_DG);
-    ytg[q] = readlane(Y[q][0], L_TG);
-    wahp[q] = readlane(w[q][0], L_AHP);
-  }
-#pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    const uint32_t ty = rd_type(rd[s]);
-    const bool qrow = ty >= R_Q0 && ty <= R_QLMAX;
-    const double iq = qrow ? rcp_nr(cx.q[rd_q(rd[s])]) : 0.0;
-    T ms[K][11], vq[K], xq[K], vb[K];
-#pragma unroll
-    for (int q = 0; q < K; ++q) {
-      slot_muls<T>(s, Y[q][s], w[q][s], from_prev(Y[q][s]), from_next(Y[q][s]), ydg[q], ytg[q], wahp[q], rs[q],
-                   ms[q]);
-      // v_q(x), x = a amnu / q
-      xq[q] = fv[q][FT_A] * fv[q][FT_AMNU] * iq;
-      vq[q] = rsqrt_t<T>(1.0 + xq[q] * xq[q]);
-      vb[q] = tconst<T>(0.0);
-    }
-    chain_feature_adj<K, T>(rd[s], cx, fv, vq, ms, acc, vb);
-    if (s == 0) {
-      T sp[K][FT_N];
-#pragma unroll
-      for (int q = 0; q < K; ++q)
-#pragma unroll
-        for (int m = 0; m < FT_N; ++m) sp[q][m] = tconst<T>(0.0);
-      special_feature_adj<K, T>(cx, fv, ms, sp);
-      if (lane == 0) {
-#pragma unroll
-        for (int q = 0; q < K; ++q)
-#pragma unroll
-          for (int m = 0; m < FT_N; ++m) acc[q][m] += sp[q][m];
-      }
-    }
-    if (qrow) {
-#pragma unroll
-      for (int q = 0; q < K; ++q) {
-        const T dvdx = -xq[q] * vq[q] * vq[q] * vq[q];
-        acc[q][FT_A] += vb[q] * dvdx * fv[q][FT_AMNU] * iq;
-        acc[q][FT_AMNU] += vb[q] * dvdx * fv[q][FT_A] * iq;
+      const double y = Y[q][s], ws = w[q][s], ndy = R.nd[s] * y, ney = R.ne[s] * y;
+      acc[q][0] = acc[q][0] + ws * (R.upi[s] * rs[q].Pi - R.ph[s] * y);
+      if ((R.qmask >> s) & 1u) {
+        T v, iv;
+        bin_velocity(F[FT_A], R.aq[s], v, iv);
+        const T x = F[FT_A] * R.aq[s];
+        const double base = ws * (from_prev(y) * R.sub[s] + from_next(y) * R.sup[s]);
+        const T g = ndy * (shi * iv - wa * (iv + v)) + ney * rs[q].se;
+        const T vb = base - ndy * (F[FT_RN] * (shi * (iv * iv) + wa * (1.0 - iv * iv)));
+        const bool qrow = rd_type(rd[s]) >= R_Q0 && rd_type(rd[s]) <= R_QLMAX;
+        acc[q][1] = acc[q][1] - vb * ((x * x) * (v * v * v));
+        acc[q][2] = acc[q][2] + sel(qrow, g, tconst<T>(0.0));
+        acc[q][3] = acc[q][3] + sel(qrow, tconst<T>(0.0), g);
+      } else {
+        acc[q][3] = acc[q][3] + (ndy * (shi - 2.0 * wa) + ney * rs[q].se);
       }
     }
   }
-  if (lane == L_A) {  // f_a = aH a, weight w_a (the leaf multiplier of the a-row)
+  double flat[8];
 #pragma unroll
-    for (int q = 0; q < K; ++q) {
-      acc[q][FT_AH] += w[q][0] * fv[q][FT_A];
-      acc[q][FT_A] += w[q][0] * fv[q][FT_AH];
+  for (int i = 0; i < 8; ++i) flat[i] = i < 4 * K * C ? comp(acc[(i / C) / 4 % K][(i / C) % 4], i % C) : 0.0;
+  wave_sum8(flat);
+#pragma unroll
+  for (int i = 0; i < 4 * K * C; ++i) comp(acc[(i / C) / 4][(i / C) % 4], i % C) = flat[i];
+  const double amnu = vval(fv[0][FT_AMNU]), iam = amnu != 0.0 ? 1.0 / amnu : 0.0;
+#pragma unroll
+  for (int q = 0; q < K; ++q) {
+    const T *F = fv[q];
+    T *o = fb[q];
+    auto y = [&](int lane) { return readlane(Y[q][0], lane); };
+    auto W = [&](int lane) { return readlane(w[q][0], lane); };
+    const T sh = rs[q].sh, se = rs[q].se;
+    const T ia = rcp_a(F[FT_A]);
+    const double wahp = W(L_AHP), wA = W(L_A), wtb = W(L_TB);
+    const double ytb = y(L_TB), ytg = y(L_TG), ytc = y(L_TC);
+    const T shi = sh * F[FT_IAH], wa = wahp * F[FT_A];
+    const double d = wtb * (ytg - ytb);  // theta_b: pb43 opac on the super- minus the diagonal
+    o[FT_OPAC] = acc[q][0] + (W(L_TG) * ytb + d * F[FT_PB43]);
+    o[FT_PB43] = d * F[FT_OPAC];
+    o[FT_CS2] = tconst<T>(wtb * y(L_DB) * k2);
+    o[FT_RN] = acc[q][2];
+    o[FT_RR] = acc[q][3];
+    o[FT_RC] = y(L_DC) * (shi - wa) + (hk2 * ytc) * se;
+    o[FT_RB] = y(L_DB) * (shi - wa) + (hk2 * ytb) * se;
+    o[FT_RG] = y(L_DG) * (shi - 2.0 * wa) + ((4.0 / 3.0) * hk2 * ytg) * se;
+    o[FT_IAH] = sh * rs[q].H * F[FT_AH];
+    o[FT_A] = (acc[q][1] + wahp * rs[q].F1) * ia + wA * F[FT_AH];  // the a-row is aH a
+    o[FT_AMNU] = acc[q][1] * iam;
+    o[FT_AH] = wA * F[FT_A] - (W(L_TC) * ytc + wtb * ytb);
+    o[FT_RQ] = tconst<T>(0.0);
+    o[FT_W] = tconst<T>(0.0);
+    o[FT_CA2] = tconst<T>(0.0);
+    o[FT_CS2Q] = tconst<T>(0.0);
+    if (!cx.lambda) {
+      const T aH = F[FT_AH], cs2Q = F[FT_CS2Q], RQ = F[FT_RQ];
+      const T opw = 1.0 + F[FT_W], dc = cs2Q - F[FT_CA2];
+      const double yq = y(L_DQ), yt = y(L_TQ), wq = W(L_DQ), wt = W(L_TQ);
+      const double dgq = wq * yq, sup = wq * yt, sub = wt * yq, dgt = wt * yt;
+      const T ce = yt * se, c1q = yq * wa, c1t = (9.0 * ik2) * (yt * wa);  // c1 multipliers times a, and 9 / k^2
+      const T g9 = (9.0 * ik2) * (aH * aH), t3 = 1.0 + 3.0 * cs2Q;
+      const T iopw = rcp_a(opw), sk = (sub * k2) * iopw;
+      const T og = opw * g9 * sup + c1t * (aH * opw * RQ);
+      // diag -3 (cs2Q - w) aH, sup -opw - 9 opw (cs2Q - ca2) aH^2 / k^2, uh -opw / 2, ch RQ / aH,
+      // c1 -a RQ (1 + 3 cs2Q); sub cs2Q k^2 / opw, diag -(1 - 3 cs2Q) aH, ceta opw RQ / 2 k^2,
+      // c1 -9 a (cs2Q - ca2) aH opw RQ / k^2
+      o[FT_CS2Q] = (3.0 * (dgt - dgq)) * aH - og - 3.0 * (c1q * RQ) + sk;
+      o[FT_CA2] = og;
+      o[FT_W] = (3.0 * dgq) * aH - sup - dc * (sup * g9 + c1t * (aH * RQ)) - (0.5 * wq) * rs[q].H - sk * cs2Q * iopw +
+                hk2 * (ce * RQ);
+      o[FT_AH] = o[FT_AH] - (3.0 * dgq) * (cs2Q - F[FT_W]) - dgt * (1.0 - 3.0 * cs2Q) -
+                 opw * dc * ((18.0 * ik2 * sup) * aH + c1t * RQ);
+      o[FT_RQ] = yq * shi - c1q * t3 + hk2 * (ce * opw) - c1t * (dc * aH * opw);
     }
   }
-#pragma unroll
-  for (int q = 0; q < K; ++q)
-#pragma unroll
-    for (int m = 0; m < FT_N; ++m) fb[q][m] += acc[q][m];
-}
-template <int NS, int K, class T = double>
-DEB_OUTLINE void feature_partials(const Ctx &cx, const uint32_t (&rd)[NS], const T (&fv_in)[K][FT_N],
-                                  const double (&Y_in)[K][NS], const double (&w_in)[K][NS],
-                                  const RowSumsT<T> (&rs_in)[K], T (&fb)[K][FT_N]) {
-  feature_partials_body<NS, K, T>(cx, rd, fv_in, Y_in, w_in, rs_in, fb);
 }
 
 // One tangent direction per lane: lane & 7 == 0 carries d/da (component 0 of
@@ -753,9 +578,7 @@ DEB_OUTLINE void acol_pass(Mode<NS> &m, Ctx &cx, dual a, double invtau, const do
     wd[0][s] = w[s];
   }
   T fb[1][FT_N];
-#pragma unroll
-  for (int q = 0; q < FT_N; ++q) fb[0][q] = tconst<T>(0.0);
-  feature_partials_body<NS, 1, T>(cx, m.rd, F, Yd, wd, rs, fb);
+  feature_totals<NS, 1, T>(cx, K, m.rd, F, Yd, wd, rs, fb);
 #pragma unroll
   for (int q = 0; q < FT_N; ++q) fb_out[q] = fb[0][q];
 }
@@ -828,13 +651,11 @@ DEB_OUTLINE void stage_rows(Ctx &cx, Mode<NS> &m, double ai, double iti, const d
 #pragma unroll
   for (int q = 0; q < FT_N; ++q) {
     fvs[1][q] = (double)fvJ_in[q];
-    fbs[0][q] = 0.0;
-    fbs[1][q] = 0.0;
   }
   // one background evaluation along a: its values for the rows, both for the features
   RowSums rsq[2];
+  const RowK<NS> K = m.rk;
   {
-    const RowK<NS> K = m.rk;
     BgCache g;
     const BgRow<dual> bd = mode_background<NS>(m, g, mkd(ai, 1.0));
     dual F[FT_N];
@@ -856,18 +677,17 @@ DEB_OUTLINE void stage_rows(Ctx &cx, Mode<NS> &m, double ai, double iti, const d
     wq[1][s] = (s == 0 && lane == L_A) ? 0.0 : rb[s];
   }
   rsq[1] = jac_sums<NS>(m, ki, wq[1]);
-  feature_partials_body<NS, 2>(cx, m.rd, fvs, Yq, wq, rsq, fbs);
+  feature_totals<NS, 2>(cx, K, m.rd, fvs, Yq, wq, rsq, fbs);
   double ga = 0.0;
 #pragma unroll
   for (int q = 0; q < FT_N; ++q) ga += dfa[q] * fbs[0][q];
-  ga = wave_sum1(ga);
   if (lane == L_A) ub[0] += ga;
 #pragma unroll
   for (int s = 0; s < NS; ++s) ub_out[s] = ub[s];
-  const double t0 = wave_sum_spread(fbs[0]), t1 = wave_sum_spread(fbs[1]);
-  if (lane < FT_N) {
-    fb_out[lane] = t0;
-    fbJ_io[lane] += t1;
+#pragma unroll
+  for (int q = 0; q < FT_N; ++q) {
+    fb_out[q] = fbs[0][q];
+    fbJ_io[q] += fbs[1][q];
   }
 }
 
@@ -1034,7 +854,6 @@ __device__ __forceinline__ void rodas5_step_vjp(Mode<NS> &m, Ctx &cx, double t0,
       for (int s = 0; s < NS; ++s) KBp(j, s) += aij * ub[s];
     }
   }
-  lds_sync();
   // the stages' input-tangent directions
   {
     const double g = lane_contract_stages(cx, cst);
@@ -1054,29 +873,20 @@ __device__ __forceinline__ void rodas5_step_vjp(Mode<NS> &m, Ctx &cx, double t0,
     ad.v = a0;
     ad.d = 1.0;
     // rho^T A'(a) (the derivative of the transposed apply), and for
-    // S = rho^T f(a, y0) the per-lane feature partials in dual arithmetic
+    // S = rho^T f(a, y0) the feature partials in dual arithmetic
     dual gy[NS], fbd[FT_N];
     acol_pass<NS>(m, cx, ad, it0, rho, y0, gy, fbd);
 #pragma unroll
     for (int s = 0; s < NS; ++s) y0b[s] += gy[s].d;
-    // the feature partials P and their a-derivative Q, summed over the wave
-    // and kept in the stage block (whose contraction has been read), then the
-    // features' second derivatives
+    // the feature partials P and their a-derivative Q, kept in the stage block
+    // (whose contraction has been read), then the features' second derivatives
     // (the J(t0, y0) k_i terms' partials join Q: contracted with the same
     // feature tangents at a0, to first order)
-    double P[FT_N], Q[FT_N];
 #pragma unroll
     for (int q = 0; q < FT_N; ++q) {
-      P[q] = fbd[q].v;
-      Q[q] = fbd[q].d;
+      cst[q] = fbd[q].v;
+      cst[FT_N + q] = fbd[q].d + fbJl[q];
     }
-    const double p = wave_sum_spread(P), q = wave_sum_spread(Q);
-    lds_sync();
-    if (lane < FT_N) {
-      cst[lane] = p;
-      cst[FT_N + lane] = q + fbJl[lane];
-    }
-    lds_sync();
     const double g = lane_contract2(cx, a0, cst);
     a0b += readlane(g, 0);
     double tl[MAXDIR];

@@ -123,10 +123,10 @@ __global__ void __launch_bounds__(WAVE) deb_rhs_vjp_kernel(const Params<NS> P_, 
     Yq[0][s] = y[s];
     wq[0][s] = w[s];
   }
-#pragma unroll
-  for (int q = 0; q < FT_N; ++q) fb[0][q] = 0.0;
-  feature_partials<NS, 1>(cx, rd, fv, Yq, wq, rs, fb);
-  wave_sum<FT_N>(fb[0]);
+  {
+    const RowK<NS> R = m.rk;
+    feature_totals<NS, 1>(cx, R, rd, fv, Yq, wq, rs, fb);
+  }
   const double gl = lane_contract(cx, a, fb[0]);
   double gth[MAXDIR];
   lane_gather(gl, H.ndir, gth);

@@ -558,6 +558,7 @@ struct RowK {
   double uh[NS], ueta[NS], upi[NS];    // where h', eta', Pi enter (upi times opac)
   double ch[NS], ceta[NS], cpi[NS];    // contributions to h', eta', Pi
   double aq[NS];                       // m_nu / q on massive-nu rows, else 0
+  double nd[NS], ne[NS];               // neutrino rows: weight of the density in ch and c1, in ceta
   double leaf, dah;                    // slot 0: leaf coupling, -aH on the diagonal
   uint32_t qmask;                      // slots that hold massive-nu rows (wave-uniform)
 };
@@ -607,6 +608,8 @@ __device__ __forceinline__ void row_consts(const uint32_t (&rd)[NS], const Ctx &
     K.ceta[s] = TR ? (4.0 / 3.0) * c.Neff * c.grhor * hk2 : (Q1 ? c.Nmnu * c.grhor * k * wq * hk2 : 0.0);
     K.cpi[s] = (F2 || G0 || G2) ? 1.0 : 0.0;
     K.aq[s] = qrow ? c.amnu * rcp_nr(cx.q[qi]) : 0.0;
+    K.nd[s] = DR ? 1.0 : (Q0 ? wq : 0.0);
+    K.ne[s] = TR ? (4.0 / 3.0) * hk2 : (Q1 ? k * wq * hk2 : 0.0);
     if (__ballot(qrow) != 0) K.qmask |= 1u << s;
     if (s == 0) {
       const double rc = c.grhom * (c.Omegam - c.Omegab), rb = c.grhom * c.Omegab;
