@@ -38,30 +38,39 @@ __global__ void __launch_bounds__(OBS_BLOCK)
 // minimum-norm solution c of A c = e_0 with A[m][j] = x_j^m, x_j = pos - j
 // (the reference's reversed grid), i.e. c = Q R^-T e_0 for the thin QR
 // factorisation A^T = Q R.  Modified Gram-Schmidt with one reorthogonalisation
-// pass on x scaled to [-1, 1] (the scaling of row m cancels in c).  One
-// thread; p + 1 <= 8 columns of length W.
+// pass on x scaled to [-1, 1] (the scaling of row m cancels in c).  The block's
+// first wave calls it; p + 1 <= 8 columns of length W, entry j on lane j % 64
+// (each lane touches its own entries of q only), the dot products summed over
+// the wave.
 __device__ void savgol_coeffs(int W, int p, double *c, double *q /* [p+1][W] */) {
+  const int lane = threadIdx.x;
   const int half = W / 2;
   const double pos = (W % 2) ? (double)half : half - 0.5;
   const double sc = pos > 0.0 ? 1.0 / pos : 1.0;
   double R[8][8];
   for (int m = 0; m <= p; ++m) {
     double *qm = q + m * W;
-    for (int j = 0; j < W; ++j) qm[j] = pow((pos - j) * sc, (double)m);
+    for (int j = lane; j < W; j += WAVE) {
+      const double x = (pos - j) * sc;
+      double v = 1.0;
+      for (int t = 0; t < m; ++t) v *= x;
+      qm[j] = v;
+    }
     for (int n = 0; n <= m; ++n) R[n][m] = 0.0;
     for (int pass = 0; pass < 2; ++pass)
       for (int n = 0; n < m; ++n) {
         const double *qn = q + n * W;
         double d = 0.0;
-        for (int j = 0; j < W; ++j) d += qn[j] * qm[j];
-        for (int j = 0; j < W; ++j) qm[j] -= d * qn[j];
+        for (int j = lane; j < W; j += WAVE) d += qn[j] * qm[j];
+        d = wave_sum1(d);
+        for (int j = lane; j < W; j += WAVE) qm[j] -= d * qn[j];
         R[n][m] += d;
       }
     double nn = 0.0;
-    for (int j = 0; j < W; ++j) nn += qm[j] * qm[j];
-    nn = sqrt(nn);
+    for (int j = lane; j < W; j += WAVE) nn += qm[j] * qm[j];
+    nn = sqrt(wave_sum1(nn));
     R[m][m] = nn;
-    for (int j = 0; j < W; ++j) qm[j] /= nn;
+    for (int j = lane; j < W; j += WAVE) qm[j] /= nn;
   }
   // z = R^-T e_0 (forward substitution with R^T, lower triangular)
   double z[8];
@@ -70,7 +79,7 @@ __device__ void savgol_coeffs(int W, int p, double *c, double *q /* [p+1][W] */)
     for (int n = 0; n < m; ++n) s -= R[n][m] * z[n];
     z[m] = s / R[m][m];
   }
-  for (int j = 0; j < W; ++j) {
+  for (int j = lane; j < W; j += WAVE) {
     double s = 0.0;
     for (int m = 0; m <= p; ++m) s += q[m * W + j] * z[m];
     c[j] = s;
@@ -118,7 +127,7 @@ __global__ void __launch_bounds__(OBS_BLOCK)
     s.P[i] = P;
     s.lp[i] = log(P);
   }
-  if (threadIdx.x == 0) savgol_coeffs(W, p, s.c, q_scratch + (int64_t)c * (p + 1) * W);
+  if (threadIdx.x < WAVE) savgol_coeffs(W, p, s.c, q_scratch + (int64_t)c * (p + 1) * W);
   __syncthreads();
   smooth_log(nk, W, s.c, s.lp, out + (int64_t)c * nk, s.P);
 }
@@ -142,7 +151,7 @@ __global__ void __launch_bounds__(OBS_BLOCK)
       th[i] = f * yc[(int64_t)i * nfield + 5];
     }
   } else {
-    if (threadIdx.x == 0) savgol_coeffs(W, p, s.c, q_scratch + (int64_t)c * (p + 1) * W);
+    if (threadIdx.x < WAVE) savgol_coeffs(W, p, s.c, q_scratch + (int64_t)c * (p + 1) * W);
     for (int pass = 0; pass < 2; ++pass) {
       const int idx = 4 + pass;
       double *dst = pass == 0 ? dl : th;
@@ -230,11 +239,8 @@ __device__ cplx lngamma_complex(cplx z) {
   return {1.14472988584940017414342735135 - ls.re - lg.re, -ls.im - lg.im};
 }
 
-// cos and sin of 2 pi m / N for integer m (reduced mod N first, so the
-// argument is exact to the rounding of one division)
-__device__ __forceinline__ cplx twiddle(int64_t m, int N) {
-  m %= N;
-  if (m < 0) m += N;
+// cos and sin of 2 pi m / N, 0 <= m < N
+__device__ __forceinline__ cplx twiddle(int m, int N) {
   double s, c;
   sincos(2.0 * PI * (double)m / (double)N, &s, &c);
   return {c, s};
@@ -244,24 +250,31 @@ __device__ __forceinline__ cplx twiddle(int64_t m, int N) {
 // f_m *= exp(2i (theta_m - log(pi) kappa_m)), kappa_m = pi m / L,
 // theta_m = Im lnGamma((1.5 + ell)/2 + i kappa_m); then
 // xi_n = Re(i^ell irfft(f)_n) / (2 pi r_n)^1.5 with r = 2 pi / k, returned
-// in reversed order (r increasing) with r
+// in reversed order (r increasing) with r.  The N twiddle factors are formed
+// once per block and kept in LDS; a sum walks them with its index reduced mod N
+// by a subtraction.
 __global__ void __launch_bounds__(OBS_BLOCK)
     deb_xi_kernel(int N, const double *k, const double *P, int ell, double *xi, double *r) {
   __shared__ double a[DEB_OBS_MAXK];
   __shared__ cplx f[DEB_OBS_MAXK / 2 + 1];
+  __shared__ cplx tw[DEB_OBS_MAXK];
   const int c = blockIdx.x;
   const double *kc = k + (int64_t)c * N;
   const double *Pc = P + (int64_t)c * N;
-  for (int i = threadIdx.x; i < N; i += blockDim.x) a[i] = Pc[i] * pow(kc[i], 1.5);
+  for (int i = threadIdx.x; i < N; i += blockDim.x) {
+    a[i] = Pc[i] * pow(kc[i], 1.5);
+    tw[i] = twiddle(i, N);
+  }
   __syncthreads();
   const double L = log(kc[N - 1] / kc[0]);
   const int M = N / 2 + 1;
   for (int m = threadIdx.x; m < M; m += blockDim.x) {
     double re = 0.0, im = 0.0;
-    for (int j = 0; j < N; ++j) {
-      const cplx w = twiddle(-(int64_t)m * j, N);
+    for (int j = 0, t = 0; j < N; ++j) {
+      const cplx w = tw[t];  // of -m j mod N
       re += a[j] * w.re;
       im += a[j] * w.im;
+      t = t < m ? t + N - m : t - m;
     }
     const double kap = PI * m / L;
     const double theta = lngamma_complex({(1.5 + ell) / 2.0, kap}).im;
@@ -275,8 +288,10 @@ __global__ void __launch_bounds__(OBS_BLOCK)
   const int e4 = ((ell % 4) + 4) % 4;  // i^ell = 1, i, -1, -i
   for (int n = threadIdx.x; n < N; n += blockDim.x) {
     double x = f[0].re;
-    for (int m = 1; m < N / 2; ++m) {
-      const cplx w = twiddle((int64_t)m * n, N);
+    for (int m = 1, t = n; m < N / 2; ++m) {
+      const cplx w = tw[t];  // of m n mod N
+      t += n;
+      t = t >= N ? t - N : t;
       x += 2.0 * (f[m].re * w.re - f[m].im * w.im);
     }
     x += f[N / 2].re * ((n & 1) ? -1.0 : 1.0);
