@@ -7,9 +7,10 @@
 //                       writes the output fields at every tau_out.
 //   deb_forward_tape_kernel  the same solve, also writing every accepted state
 //                       to the checkpoint tape of the gradient path.
-//   deb_forward_batched_kernel  one wavefront per (cosmology, group of
+//   deb_forward_batched_kernel  one workgroup per (cosmology, group of
 //                       batch_size consecutive k): the group shares one step
-//                       sequence (evolve_perturbations_batched).
+//                       sequence (evolve_perturbations_batched), its modes
+//                       are spread over the workgroup's waves.
 //   deb_rhs_kernel      test hook: model_synchronous for given states.
 //   deb_step_kernel     test hook: one Rodas5Transformed step.
 #include <hip/hip_runtime.h>
@@ -22,6 +23,7 @@
 #include <string>
 #include <vector>
 
+#include "deb_batch.h"
 #include "deb_forward.h"
 #include "deb_kargs.h"
 #include "deb_host.h"
@@ -77,19 +79,21 @@ __global__ void __launch_bounds__(WAVE) deb_forward_kernel(const Params<NS> P_) 
   integrate_mode<NS>(P, ci, ki, lds, (lds_double *)pcr);
 }
 
-// evolve_perturbations_batched: one wavefront per (cosmology, group of B
-// consecutive k), groups of the largest k first.
-template <int NS>
-__global__ void __launch_bounds__(WAVE) deb_forward_batched_kernel(const Params<NS> P_, const int B, double *ws) {
+// evolve_perturbations_batched: one workgroup of up to NW waves per (cosmology,
+// group of B consecutive k), groups of the largest k first.
+template <int NS, int NW>
+__global__ void __launch_bounds__(NW * WAVE)
+    deb_forward_batched_kernel(const Params<NS> P_, const int B, double *ws) {
   const Params<NS> &P = kernel_params<NS>();
-  __shared__ double lds[fwd_lds_doubles<NS>()];
-  __shared__ double pcr[pcr_lds_doubles<NS>()];
+  __shared__ BatchWave<NS> waves[NW];
+  __shared__ BatchShare<NW> share;
   const int ng = P.nk / B;
   const int item = blockIdx.x;
   if (item >= P.n_cosmo * ng) return;
   const int g = ng - 1 - item / P.n_cosmo;
   const int ci = item % P.n_cosmo;
-  integrate_batch<NS>(P, ci, g * B, B, lds, (lds_double *)pcr, ws);
+  const int w = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / WAVE);
+  integrate_batch<NS, NW>(P, ci, g * B, B, w, (int)blockDim.x / WAVE, waves[w], share, ws);
 }
 
 // The forward solve that also writes every accepted state to the checkpoint
@@ -237,8 +241,14 @@ int run_forward_batched(const deb_config_t *cfg, const Layout &L, int n_cosmo, c
   P.status = status;
   P.nsteps = nsteps;
   const unsigned items = (unsigned)((int64_t)n_cosmo * (nk / batch));
-  hipLaunchKernelGGL(deb_forward_batched_kernel<NS>, dim3(items), dim3(WAVE), 0, st, P, batch,
-                     static_cast<double *>(ws));
+  // groups of one keep a single wave's LDS per workgroup
+  const dim3 block((unsigned)(batch_waves_of(batch_waves<NS>(), batch) * WAVE));
+  if (batch == 1)
+    hipLaunchKernelGGL((deb_forward_batched_kernel<NS, 1>), dim3(items), block, 0, st, P, batch,
+                       static_cast<double *>(ws));
+  else
+    hipLaunchKernelGGL((deb_forward_batched_kernel<NS, batch_waves<NS>()>), dim3(items), block, 0, st, P, batch,
+                       static_cast<double *>(ws));
   return hip_check(hipGetLastError(), "batched forward kernel launch");
 }
 
