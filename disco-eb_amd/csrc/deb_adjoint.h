@@ -812,11 +812,6 @@ __device__ __forceinline__ void rodas5_step_vjp(Mode<NS> &m, Ctx &cx, double t0,
         }
       }
     }
-    for (int j = 0; j < i; ++j) {
-      const double cij = kC[i][j];
-#pragma unroll
-      for (int s = 0; s < NS; ++s) KBp(j, s) += (cij * ih) * rb[s];
-    }
     const double ti = t0 + kc[i] * h;
     const double iti = 1.0 / ti;
     // dot products: h-derivative of W, C/h and d h dT terms; explicit time
@@ -848,11 +843,24 @@ __device__ __forceinline__ void rodas5_step_vjp(Mode<NS> &m, Ctx &cx, double t0,
     }
 #pragma unroll
     for (int s = 0; s < NS; ++s) y0b[s] += ub[s];
-    for (int j = 0; j < i; ++j) {
-      const double aij = kA[i][j];
+    // cotangents of the earlier stages, in two batches (those of this stage on
+    // have been read, and their tableau entries are zero)
+    auto feed = [&](auto first, auto count) {
+      constexpr int J0 = decltype(first)::value, NJ = decltype(count)::value;
+      double kb[NJ][NS];
 #pragma unroll
-      for (int s = 0; s < NS; ++s) KBp(j, s) += aij * ub[s];
-    }
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int s = 0; s < NS; ++s) kb[j][s] = KBp(J0 + j, s);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const double aij = kA[i][J0 + j], cij = kC[i][J0 + j] * ih;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) KBp(J0 + j, s) = kb[j][s] + (cij * rb[s] + aij * ub[s]);
+      }
+    };
+    feed(std::integral_constant<int, 0>{}, std::integral_constant<int, 3>{});
+    if (i > 3) feed(std::integral_constant<int, 3>{}, std::integral_constant<int, 4>{});
   }
   // the stages' input-tangent directions
   {

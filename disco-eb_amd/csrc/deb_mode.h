@@ -172,7 +172,8 @@ struct Coef {
 enum : int { C_SUB = 0, C_DIAG, C_SUP, C_UH, C_UETA, C_UPI, C_CH, C_CETA, C_CPI, C_C1, C_LEAF };
 
 // The coefficient fields of one row (model_synchronous, perturbations.py:
-// 84-371), each passed to sink(field, value).  Every case sets each of its
+// 84-371): the equations row by row, with the wave form below the reference
+// that the host emulation checks; the kernels run row_lin.  Each is passed to sink(field, value).  Every case sets each of its
 // fields once.  The formulas use the evaluation's reciprocals (b.ia, b.ia2,
 // b.iaH) and per-mode constants, so a case body holds multiplications only:
 // the divergent switch runs every case present in a slot, and a division per
