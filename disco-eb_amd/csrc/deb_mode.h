@@ -645,9 +645,8 @@ __device__ __forceinline__ dual sel(bool c, dual x, dual y) { return {c ? x.v : 
 
 // log x for positive normal x, NaN otherwise: x = m 2^e with m in
 // [1/sqrt 2, sqrt 2], log m = 2 atanh z, z = (m - 1) / (m + 1), |z| < 0.172,
-// by its series up to z^23 (remainder below 1e-19); about one ulp of log x
-// where e != 0, 2e-16 absolute elsewhere.  A third of the instructions of the
-// library's log, which carries the result to less than an ulp.
+// by its series up to z^23 (remainder below 1e-19); within about an ulp of
+// log x.  Two fifths of the instructions of the library's log.
 __device__ __forceinline__ double log_pos(double x) {
   const int hi = __double2hiint(x);
   int e = (hi >> 20) - 1023;
@@ -655,7 +654,9 @@ __device__ __forceinline__ double log_pos(double x) {
   const bool up = m > 1.4142135623730951;
   m = up ? 0.5 * m : m;
   e = up ? e + 1 : e;
-  const double z = (m - 1.0) * rcp_nr(m + 1.0), w = z * z;
+  // (the quotient corrected by its residual, the rounding of m + 1 included)
+  const double f = m - 1.0, d1 = m + 1.0, rd = rcp_nr(d1), z0 = f * rd;
+  const double z = fma(fma(-z0, d1, f) - z0 * (m - (d1 - 1.0)), rd, z0), w = z * z;
   double p = 2.0 / 23.0;
   p = fma(p, w, 2.0 / 21.0);
   p = fma(p, w, 2.0 / 19.0);
