@@ -351,7 +351,7 @@ DEB_OUTLINE RowSums coef_pass(Mode<NS> &m, Ctx &cx, double a, double invtau, con
 // feature; the remaining rows sit on fixed lanes of slot 0 and are combined as
 // wave-uniform values read from there.  (Summed as 16 features per contraction
 // from per-row multipliers, a stage's two contractions took 2400 instructions;
-// this form takes about 700.)
+// this form takes about 700: gradient of 256 k at lmax 32 132 -> 108 ms.)
 template <int NS, int K, class T = double>
 __device__ __forceinline__ void feature_totals(const Ctx &cx, const RowK<NS> &R, const uint32_t (&rd)[NS],
                                                const T (&fv)[K][FT_N], const double (&Y)[K][NS],
@@ -628,6 +628,11 @@ __device__ __forceinline__ RowSums jac_sums(const Mode<NS> &m, const double (&Y)
   return RowSums{part[0], part[1], part[2], part[3], part[4], part[5], part[6]};
 }
 
+// (Bound by the latency of the step factors and row constants in the caller's
+// frame and by instruction issue.  With the rows from the mode's constants and
+// one background evaluation for rows and features the gradient of 256 k at lmax
+// 32 went from 160 to 136 ms; inlined into the stage loop it measured 133 ms
+// where the call takes 112.)
 // The row work of one reverse stage as a single call: the transposed row pass
 // at the stage point (ub = J(t_i, u_i)^T rb, the stage's features and their
 // a-derivative dfa), the row sums of the J(t0, y0) k_i term, and the feature

@@ -11,7 +11,8 @@ namespace deb {
 // norm; one wave stepping all 16 modes of the default batch in turn left a
 // launch of 8 groups on 8 of the chip's 1024 SIMDs.  Two waves per SIMD fit the
 // LDS of a CU up to two slots (18 KB per wave), one wave per SIMD above
-// (37 KB).
+// (37 KB).  128 k in groups of 16 at lmax 11: 198 ms on one wave per group, 50.5
+// ms on eight.
 template <int NS>
 constexpr int batch_waves() {
   return NS <= 2 ? 8 : 4;

@@ -406,7 +406,10 @@ __constant__ double kd[8] = {R5::d1, R5::d2, R5::d3, R5::d4, R5::d5, 0.0, 0.0, 0
 // one Rodas5Transformed step (ode_integrators_stiff.py:718-834): y1 and err = k8;
 // st(i, k) sees every stage vector k_{i+1} once it is solved.  The stages run
 // as a loop over the tableau: unrolled, the step is about 240 KB of code, four
-// times the instruction cache, and every wave fetched it again each step.
+// times the instruction cache, and every wave fetched it again each step.  A
+// single wave's instruction issue bounds it now (64 cosmologies x 256 k at lmax
+// 32: 384 ms unrolled, 227 ms as a loop with the rows as constants, 146 ms with
+// the register-held background and the split sums).
 // Stage 1's right-hand side is the factorisation's.  With kl (the wave's LDS,
 // 7 x NS x 64 doubles) the stage vectors k1..k7 are kept there, else in
 // registers.
