@@ -23,6 +23,19 @@ inline int batch_waves_of(int cap, int B) {
   const int rounds = (B + cap - 1) / cap;
   return (B + rounds - 1) / rounds;
 }
+// Waves of the kernel instance that runs w of them: an instance reserves the LDS
+// of all its waves, so it is the smallest that holds them.  Up to four waves a
+// lane has 512 registers, one wave per SIMD runs at a time, and with its waves'
+// LDS a CU holds 4 / w groups.  The eight-wave instance (256 registers, spills
+// at two slots) is for five waves and more, and at one slot for three and four
+// too: there a wave's state is small enough that two waves per SIMD in 256
+// registers beat one.  2048 groups at two slots: 2 k 5.5 ms, 4 k 11.0 ms (14.4
+// and 17.9 ms on the eight-wave instance; one wave per group before the present
+// step 12.2 and 24.2); at one slot 4 k 5.8 ms, on a four-wave instance 8.9.
+template <int NS>
+constexpr int batch_instance(int w) {
+  return w <= 1 ? 1 : (w <= 2 ? 2 : (NS > 1 && w <= 4 ? 4 : 8));
+}
 
 // one wave's LDS
 template <int NS>

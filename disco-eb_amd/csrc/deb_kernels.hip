@@ -79,8 +79,8 @@ __global__ void __launch_bounds__(WAVE) deb_forward_kernel(const Params<NS> P_) 
   integrate_mode<NS>(P, ci, ki, lds, (lds_double *)pcr);
 }
 
-// evolve_perturbations_batched: one workgroup of up to NW waves per (cosmology,
-// group of B consecutive k), groups of the largest k first.
+// evolve_perturbations_batched: one workgroup of up to NW waves (batch_instance)
+// per (cosmology, group of B consecutive k), groups of the largest k first.
 template <int NS, int NW>
 __global__ void __launch_bounds__(NW * WAVE)
     deb_forward_batched_kernel(const Params<NS> P_, const int B, double *ws) {
@@ -241,14 +241,19 @@ int run_forward_batched(const deb_config_t *cfg, const Layout &L, int n_cosmo, c
   P.status = status;
   P.nsteps = nsteps;
   const unsigned items = (unsigned)((int64_t)n_cosmo * (nk / batch));
-  // groups of one keep a single wave's LDS per workgroup
-  const dim3 block((unsigned)(batch_waves_of(batch_waves<NS>(), batch) * WAVE));
-  if (batch == 1)
-    hipLaunchKernelGGL((deb_forward_batched_kernel<NS, 1>), dim3(items), block, 0, st, P, batch,
-                       static_cast<double *>(ws));
-  else
-    hipLaunchKernelGGL((deb_forward_batched_kernel<NS, batch_waves<NS>()>), dim3(items), block, 0, st, P, batch,
-                       static_cast<double *>(ws));
+  const int waves = batch_waves_of(batch_waves<NS>(), batch);
+  auto launch = [&](auto nw) {
+    constexpr int NW = decltype(nw)::value;
+    if constexpr (NW == batch_instance<NS>(NW) && NW <= batch_waves<NS>())
+      hipLaunchKernelGGL((deb_forward_batched_kernel<NS, NW>), dim3(items), dim3((unsigned)(waves * WAVE)), 0, st, P,
+                         batch, static_cast<double *>(ws));
+  };
+  switch (batch_instance<NS>(waves)) {
+    case 1: launch(std::integral_constant<int, 1>{}); break;
+    case 2: launch(std::integral_constant<int, 2>{}); break;
+    case 4: launch(std::integral_constant<int, 4>{}); break;
+    default: launch(std::integral_constant<int, 8>{}); break;
+  }
   return hip_check(hipGetLastError(), "batched forward kernel launch");
 }
 
