@@ -172,12 +172,10 @@ struct Coef {
 enum : int { C_SUB = 0, C_DIAG, C_SUP, C_UH, C_UETA, C_UPI, C_CH, C_CETA, C_CPI, C_C1, C_LEAF };
 
 // The coefficient fields of one row (model_synchronous, perturbations.py:
-// 84-371): the equations row by row, with the wave form below the reference
-// that the host emulation checks; the kernels run row_lin.  Each is passed to sink(field, value).  Every case sets each of its
-// fields once.  The formulas use the evaluation's reciprocals (b.ia, b.ia2,
-// b.iaH) and per-mode constants, so a case body holds multiplications only:
-// the divergent switch runs every case present in a slot, and a division per
-// case multiplied its cost.
+// 84-371), each passed to sink(field, value): the equations as they are
+// written, one case per row type, each case setting each of its fields once.
+// No kernel runs this form or row_coef_wave below; it is what the host
+// emulation checks the kernels' form (row_consts, row_lin) against, row by row.
 template <typename T, class Sink>
 __device__ __forceinline__ void row_visit(uint32_t d, const Bg<T> &b, const Ctx &cx, double invtau, Sink sink) {
   using P = ParT<T>;
@@ -402,9 +400,9 @@ __device__ __forceinline__ Coef<T> row_coef(uint32_t d, const Bg<T> &b, const Ct
 
 // row_coef organised for the wave instead of as a divergent switch, with the
 // same formulas in the same operation order (the host emulation compares the
-// two): the chain rows (hierarchies, any slot) by per-lane selects among their
-// formulas; with slot0, the fixed-lane rows of slot 0 as wave-uniform values
-// selected by lane.
+// two; no kernel runs it): the chain rows (hierarchies, any slot) by per-lane
+// selects among their formulas; with slot0, the fixed-lane rows of slot 0 as
+// wave-uniform values selected by lane.
 template <typename T>
 __device__ __forceinline__ Coef<T> row_coef_wave(uint32_t d, const Bg<T> &b, const Ctx &cx, double invtau,
                                                  bool slot0) {
@@ -550,7 +548,7 @@ __device__ __forceinline__ Coef<T> row_coef_wave(uint32_t d, const Bg<T> &b, con
 // formed once per mode (row_consts) and a right-hand side costs about a dozen
 // multiplications per slot, where the selects of row_coef_wave took about two
 // hundred instructions.  The same products as row_visit up to the order of the
-// factors.
+// factors (within 2 units of 2^-52 of it on every row).
 template <int NS>
 struct RowK {
   double sub[NS], sup[NS];             // neighbours (times v_q on massive-nu rows)
