@@ -29,9 +29,11 @@ struct Worst {
   // error of x against ref in units of EPS * scale; equal values need no scale
   void add(int which, double x, double ref, double scale) {
     ++n;
-    if (x == ref) return;
-    const double e = std::fabs(x - ref) / (EPS * scale);
-    if (!(e <= w[which])) w[which] = e;  // (NaN too)
+    if (x != ref) merge(which, std::fabs(x - ref) / (EPS * scale));
+  }
+  // a NaN stays
+  void merge(int which, double e) {
+    if (w[which] == w[which] && !(e <= w[which])) w[which] = e;
   }
 };
 
@@ -156,8 +158,7 @@ int run(simt::Input &in, const char *path) {
   Worst all;
   for (const Worst &l : lanes) {
     all.n += l.n;
-    for (int i = 0; i < 4; ++i)
-      if (!(l.w[i] <= all.w[i])) all.w[i] = l.w[i];
+    for (int i = 0; i < 4; ++i) all.merge(i, l.w[i]);
   }
   FILE *out = fopen(path, "wb");
   if (!out) return 2;

@@ -57,3 +57,42 @@ def test_cosmologies_and_instances(gpu, two, lay, batch):
         assert np.all(ref["status"] == 0) and np.array_equal(ns[c], ref["nsteps"])
         for f in (4, 6, 8, 10, 12):
             assert np.abs(y[c, :, :, f] / ref["y"][:, :, f] - 1).max() < 1e-8, (c, f)
+
+
+@pytest.mark.parametrize("lay,batch", [(SMALL, 2), (SMALL, 9), (SMALL, 16), (LARGE, 5)])
+def test_groups_that_reach_the_step_limit(gpu, two, lay, batch):
+    """A limit that some groups end below and others reach between two outputs: every mode of a group has the group's
+    status and step count, unreached outputs hold inf, what was reached is the unlimited run's to the bit."""
+    conf = dict(rtol=1e12, atol=1e12, factormax=1.15)
+    cfg = packing.make_config(max_steps=4096, **conf, **lay)
+    k, tau = _inputs(two, cfg, 3 * batch, [0.02, 0.1])
+    y, st, ns = _solve(two[0], cfg, k, tau, batch)
+    assert np.all(st == 0)
+    limit = int(ns.max()) - 1
+    assert limit > ns.min()
+    cfg = packing.make_config(max_steps=limit, **conf, **lay)
+    yl, sl, nl = _solve(two[0], cfg, k, tau, batch)
+    over = ns > limit
+    assert np.array_equal(sl, np.where(over, packing.STATUS_MAX_STEPS, packing.STATUS_OK))
+    assert np.array_equal(nl, np.minimum(ns, limit))
+    assert np.array_equal(yl[~over], y[~over])
+    assert np.array_equal(yl[over][:, 0], y[over][:, 0]) and np.all(np.isposinf(yl[over][:, 1]))
+
+
+@pytest.mark.parametrize("lay,batch,bad", [(SMALL, 2, 1), (SMALL, 4, 2), (SMALL, 9, 3), (SMALL, 16, 15), (LARGE, 5, 4)])
+def test_group_with_a_nonfinite_mode(gpu, two, lay, batch, bad):
+    """A mode of a wave other than the first without finite values rejects every step of its group until the step no
+    longer advances; the other groups are unchanged to the bit."""
+    cfg = packing.make_config(rtol=1e12, atol=1e12, factormax=1.15, factormin=1e-6, max_steps=4096, **lay)
+    k, tau = _inputs(two, cfg, 3 * batch, [0.02, 0.1])
+    y, st, _ = _solve(two[0], cfg, k, tau, batch)
+    assert np.all(st == 0)
+    kb = k.copy()
+    kb[1, batch + bad] = np.nan
+    yb, sb, nb = _solve(two[0], cfg, kb, tau, batch)
+    hit = np.zeros(k.shape, bool)
+    hit[1, batch:2 * batch] = True
+    ref = oracle.Problem(two[1][1], cfg).evolve_batched(kb[1, batch:2 * batch], tau[1], batch, nthreads=2)
+    assert np.array_equal(sb[hit], ref["status"]) and np.array_equal(nb[hit], ref["nsteps"])
+    assert np.all(sb[hit] == packing.STATUS_NONFINITE) and np.all(np.isposinf(yb[hit]))
+    assert np.all(sb[~hit] == 0) and np.array_equal(yb[~hit], y[~hit])
