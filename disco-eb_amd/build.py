@@ -18,7 +18,6 @@ SOURCES = ["deb_kernels.hip", "deb_adjoint.hip", "deb_observables.hip"]
 # kernel body (thousands of spilled registers) gave build-dependent wrong
 # reverse steps at -O3 and at -O1.
 OPT = {"deb_kernels.hip": "-O3", "deb_adjoint.hip": "-O3", "deb_observables.hip": "-O3"}
-HEADERS = ["deb_device.h", "deb_mode.h", "deb_solver.h", "deb_forward.h", "deb_host.h", "deb_adjoint.h", "deb_kargs.h"]
 FLAGS = ["--offload-arch=gfx950", "-std=c++17", "-fPIC",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wno-unused-command-line-argument"]
