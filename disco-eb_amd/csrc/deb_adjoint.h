@@ -33,12 +33,6 @@ using TD = dn<1 + MAXDIR>;          // (a or tau, theta_1..theta_MAXDIR)
 // device-assembly test of the build checks this for every outlined function.
 #define DEB_OUTLINE __device__ __noinline__
 
-__device__ __forceinline__ void lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
 // ---------------------------------------------------------------------------
 // cross-lane moves and reductions of composite scalars, component by
 // component (member access only)
@@ -696,18 +690,6 @@ DEB_OUTLINE void stage_rows(Ctx &cx, Mode<NS> &m, double ai, double iti, const d
   }
 }
 
-// per-lane multiplier of the explicit tau dependence (hierarchy truncations):
-// d f_row / d tau = trunc_row / tau^2 * y_row with trunc_row = l + 1
-template <int NS>
-__device__ __forceinline__ void trunc_weights(const uint32_t (&rd)[NS], double (&tw)[NS]) {
-#pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    const uint32_t t = rd_type(rd[s]);
-    const bool trunc = (t == R_FLMAX) | (t == R_GLMAX) | (t == R_FRLMAX) | (t == R_QLMAX);
-    tw[s] = trunc ? (rd_l(rd[s]) + 1.0) : 0.0;
-  }
-}
-
 __device__ __forceinline__ TD seed_td(double v, double d0) {
   TD r;
   r = v;
@@ -747,8 +729,10 @@ __device__ __forceinline__ void rodas5_step_vjp(Mode<NS> &m, Ctx &cx, double t0,
   __shared__ double cst_[8 * (1 + FT_N)];
   lds_double *const cst = (lds_double *)cst_;
   factor_call<NS>(m, t0, y0, h);
+  // explicit tau dependence (hierarchy truncations): d f_row / d tau = tw / tau^2 * y_row
   double tw[NS];
-  trunc_weights<NS>(m.rd, tw);
+#pragma unroll
+  for (int s = 0; s < NS; ++s) tw[s] = m.rk.tr[s];
   const double it0 = 1.0 / t0;
   const double a0 = readlane(y0[0], L_A);
   double dT[NS];
@@ -1082,7 +1066,7 @@ __device__ __forceinline__ void output_vjp(const Params<NS> &P, Ctx &cx, const A
 #pragma unroll
   for (int s = 0; s < NS; ++s)
     if (rd_type(rd[s]) != R_NONE) ls[rd_idx(rd[s])] = yo[s];
-  lds_sync();
+  BlockSync()();
   double om[DEB_NOUT_FIELDS];
 #pragma unroll
   for (int f = 0; f < DEB_NOUT_FIELDS; ++f) om[f] = w[f];
@@ -1107,10 +1091,10 @@ __device__ __forceinline__ void output_vjp(const Params<NS> &P, Ctx &cx, const A
                           L0, L1, L2, P.nq, P.n, [&](int f, const dual &v) { acc = acc + v * om[f]; });
     lg[seed] = acc.d;
   }
-  lds_sync();
+  BlockSync()();
 #pragma unroll
   for (int s = 0; s < NS; ++s) yb[s] = rd_type(rd[s]) != R_NONE ? lg[rd_idx(rd[s])] : 0.0;
-  lds_sync();
+  BlockSync()();
 }
 
 // one (cosmology, k) item of the gradient kernel.  ring: this wave's ring

@@ -101,7 +101,7 @@ __global__ void __launch_bounds__(WAVE) deb_rhs_vjp_kernel(const Params<NS> P_, 
   Ctx cx;
   hook_ctx<NS>(cx, P, H, item);
   uint32_t rd[NS];
-  double y[NS], w[NS], yb[NS], tw[NS];
+  double y[NS], w[NS], yb[NS];
   const double *ys = H.y + (long long)item * P.n, *ws = H.wbar + (long long)item * P.n;
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
@@ -132,10 +132,9 @@ __global__ void __launch_bounds__(WAVE) deb_rhs_vjp_kernel(const Params<NS> P_, 
   lane_gather(gl, H.ndir, gth);
   const double ga = readlane(gl, 0);
   if (lane == L_A) yb[0] += ga;
-  trunc_weights<NS>(rd, tw);
   double pt = 0.0;
 #pragma unroll
-  for (int s = 0; s < NS; ++s) pt += w[s] * tw[s] * it * it * y[s];
+  for (int s = 0; s < NS; ++s) pt += w[s] * m.rk.tr[s] * it * it * y[s];
   pt = wave_sum1(pt);
   double *yo = H.ybar + (long long)item * P.n;
 #pragma unroll
