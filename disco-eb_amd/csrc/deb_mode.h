@@ -643,10 +643,8 @@ __device__ __forceinline__ dual sel(bool c, dual x, dual y) { return {c ? x.v : 
 
 // log x for positive normal x, NaN otherwise: x = m 2^e with m in
 // [1/sqrt 2, sqrt 2], log m = 2 atanh z, z = (m - 1) / (m + 1), |z| < 0.172,
-// by its series up to z^23 (remainder below 1e-19).  Two fifths of the
-// instructions of the library's log.  The quotient's and the leading sum's
-// rounding errors are added to the small terms: within 0.55 ulp (the library's
-// log on the device 0.64; 1.02 with the quotient's error rounded into z).
+// by its series up to z^23 (remainder below 1e-19); within about an ulp of
+// log x.  Two fifths of the instructions of the library's log.
 __device__ __forceinline__ double log_pos(double x) {
   const int hi = __double2hiint(x);
   int e = (hi >> 20) - 1023;
@@ -654,9 +652,9 @@ __device__ __forceinline__ double log_pos(double x) {
   const bool up = m > 1.4142135623730951;
   m = up ? 0.5 * m : m;
   e = up ? e + 1 : e;
-  // z = z0 + zl, z0 the rounded quotient (the residual holds the rounding of m + 1 too)
+  // (the quotient corrected by its residual, the rounding of m + 1 included)
   const double f = m - 1.0, d1 = m + 1.0, rd = rcp_nr(d1), z0 = f * rd;
-  const double zl = (fma(-z0, d1, f) - z0 * (m - (d1 - 1.0))) * rd, w = z0 * z0;
+  const double z = fma(fma(-z0, d1, f) - z0 * (m - (d1 - 1.0)), rd, z0), w = z * z;
   double p = 2.0 / 23.0;
   p = fma(p, w, 2.0 / 21.0);
   p = fma(p, w, 2.0 / 19.0);
@@ -669,10 +667,8 @@ __device__ __forceinline__ double log_pos(double x) {
   p = fma(p, w, 2.0 / 5.0);
   p = fma(p, w, 2.0 / 3.0);
   const double d = (double)e;
-  // ln 2 in the two parts that fdlibm publishes, the first exact in products with e
-  const double l2 = d * 6.93147180369123816490e-01, s = fma(2.0, z0, l2);
-  const double t = fma(z0 * w, p, fma(2.0, zl, d * 1.90821492927058770002e-10));
-  const double r = s + (t + fma(2.0, z0, l2 - s));
+  // ln 2 in two parts, the first exact in products with e
+  const double r = fma(d, 6.93147180369123816490e-01, fma(2.0, z, fma(z * w, p, d * 1.90821492927058770002e-10)));
   return x >= 2.2250738585072014e-308 && x <= 1.7976931348623157e308 ? r : __builtin_nan("");
 }
 

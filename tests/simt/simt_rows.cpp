@@ -4,8 +4,6 @@
 // like simt_host (64 host threads per wavefront, sanitizers).  Test
 // infrastructure only.
 //
-//   simt_rows log <in.bin> <out.bin>
-//     double x[] to double log_pos(x)[]
 //   simt_rows <in.bin> <out.bin>
 //
 // in.bin: written by _write of tests/test_simt_host.py, mode 0, followed by
@@ -170,24 +168,11 @@ int run(simt::Input &in, const char *path) {
   return 0;
 }
 
-int run_log(const char *from, const char *to) {
-  FILE *in = fopen(from, "rb"), *out = fopen(to, "wb");
-  if (!in || !out) return 2;
-  double x;
-  while (fread(&x, 8, 1, in) == 1) {
-    x = log_pos(x);
-    fwrite(&x, 8, 1, out);
-  }
-  fclose(in);
-  return fclose(out);
-}
-
 }  // namespace
 
 int main(int argc, char **argv) {
-  if (argc == 4 && std::strcmp(argv[1], "log") == 0) return run_log(argv[2], argv[3]);
   if (argc != 3) {
-    fprintf(stderr, "usage: simt_rows [log] in.bin out.bin\n");
+    fprintf(stderr, "usage: simt_rows in.bin out.bin\n");
     return 2;
   }
   simt::Input in(argv[1]);

@@ -58,25 +58,3 @@ def test_rows_and_background(rows, test_param, grad_inputs, tmp_path):
         raw = (tmp_path / f"{name}.out").read_bytes()
         worst, n = np.frombuffer(raw[:32]), np.frombuffer(raw[32:], np.int32)[0]
         assert n > 0 and np.all(worst <= BOUNDS), (name, worst)
-
-
-def test_log(rows, tmp_path):
-    """log a of the background against 64-bit mantissas: half an ulp of the last sum, 0.05 for the small terms' own
-    roundings (at most 1 % of the result, a few roundings each) and 0.05 for the second order of the quotient's
-    correction: 0.6 ulp.  Over the scale factors, around powers of two and the mantissa's switch at sqrt 2, next to 1,
-    and over the whole range; NaN where there is no finite log of a normal number."""
-    assert np.finfo(np.longdouble).nmant >= 63
-    rng = np.random.default_rng(7)
-    near = np.concatenate([c * (1.0 + np.ldexp(rng.uniform(-1, 1, 4000), -rng.integers(1, 53, 4000)))
-                           for c in (1.0, 0.5, 2.0, np.sqrt(2.0), np.sqrt(0.5), 2.0**-40)])
-    x = np.concatenate([np.exp(rng.uniform(-20, 1, 300000)), rng.uniform(0.5, 1.5, 300000), near,
-                        np.ldexp(rng.uniform(1, 2, 20000), rng.integers(-1022, 1024, 20000)),
-                        [2.0**-1022, np.finfo(float).max, 1.0, np.nextafter(1, 0), np.nextafter(1, 2)]])
-    odd = np.array([0.0, -0.0, -1.0, -np.inf, np.inf, np.nan, 5e-324, np.nextafter(2.0**-1022, 0)])
-    np.concatenate([x, odd]).tofile(tmp_path / "x")
-    subprocess.run([rows, "log", str(tmp_path / "x"), str(tmp_path / "y")], check=True)
-    y = np.fromfile(tmp_path / "y")
-    ref = np.log(x.astype(np.longdouble))
-    err = np.abs((y[:x.size] - ref) / np.spacing(np.abs(ref.astype(float))))
-    assert np.all(err <= 0.6), (float(err.max()), x[np.argmax(err)])
-    assert np.all(np.isnan(y[x.size:]))
